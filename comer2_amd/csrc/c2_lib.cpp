@@ -109,6 +109,8 @@ int cbp_create(int device, size_t mem_budget, int area, cbp_handle** out)
         delete h;
         return CBP_ERR_HIP;
     }
+    int ncu = 0;
+    if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, device) == hipSuccess && ncu > 0) h->ncu = ncu;
     /* the allocation-free entry point's scratch array: its address on this
      * device (a failed lookup is reported by that entry point) */
     (void)c2_noalloc_init(device);
@@ -278,33 +280,88 @@ int c2_append_query(cbp_handle* h, const cbp_profiles* one, int32_t* qidx)
     return CBP_OK;
 }
 
-/* segments of whole profiles of about seg_cols columns each (the unit of
- * work of one phase-1 wave) */
-int c2_build_segments(cbp_handle* h, const cbp_profiles* s)
+/* the segment width for nq queries: seg_cols, or less when the chunk is too
+ * small to give every wave slot of the device (8 per CU: the column rings
+ * fill the LDS) work to balance.  One query takes two segments per slot: one
+ * leaves the slots unequal by up to a long profile, more add 63 fill steps
+ * each (schedules of log-normal databases, 30-3000 columns: two are within
+ * 16% of the bound at 7.5 M positions and 5% at 50 M, where 4096 columns are
+ * 64% and 7% off; below 4 M the longest profile is the bound).  A batch's
+ * queue takes eight tiles per slot.  One query of 150 rows against 2,000
+ * profiles ran 13 workgroups at 4096 columns (4.73 ms) */
+static int64_t seg_target(const cbp_handle* h, int64_t npos, int nq)
 {
-    h->seg_p.clear();
-    h->seg_p.push_back(0);
+    const int64_t slots = (int64_t)8 * h->ncu;
+    const int64_t one = npos / (2 * slots);
+    const int64_t t = nq > 1 ? std::max(one, npos * nq / (8 * slots)) : one;
+    return std::max<int64_t>(64, std::min<int64_t>(h->seg_cols, t));
+}
+
+static int build_segset(cbp_handle* h, const cbp_profiles* s, int64_t target, SegSet* g)
+{
+    g->target = target;
+    std::vector<std::pair<int32_t, int32_t>> v;
     int64_t acc = 0;
+    int32_t p0 = 0;
     for (int32_t p = 0; p < s->nprof; p++) {
         acc += s->len[p];
-        if (acc >= h->seg_cols) { h->seg_p.push_back(p + 1); acc = 0; }
+        if (acc >= target || p + 1 == s->nprof) { v.emplace_back(p0, p + 1); p0 = p + 1; acc = 0; }
     }
-    if (h->seg_p.back() != s->nprof) h->seg_p.push_back(s->nprof);
-    h->nseg = (int32_t)h->seg_p.size() - 1;
-    h->seg_maxcols = 0;
+    auto cols = [&](const std::pair<int32_t, int32_t>& x) {
+        return (int64_t)s->dist[x.second - 1] + s->len[x.second - 1] - (int64_t)s->dist[x.first];
+    };
+    /* widest first: a workgroup's segments are of a kind whatever order the
+     * database has, and the last workgroups to start are the shortest */
+    std::stable_sort(v.begin(), v.end(), [&](const auto& x, const auto& y) { return cols(x) > cols(y); });
+    g->nseg = (int32_t)v.size();
+    g->maxcols = (int32_t)cols(v[0]);
+    g->b.resize(v.size()); g->e.resize(v.size());
+    for (size_t i = 0; i < v.size(); i++) { g->b[i] = v[i].first; g->e[i] = v[i].second; }
+    int rc;
+    if ((rc = dupload(h, g->db, g->b.data(), g->b.size()))) return rc;
+    if ((rc = dupload(h, g->de, g->e.data(), g->e.size()))) return rc;
+    HIPCHK(hipStreamSynchronize(h->stream));
+    return CBP_OK;
+}
+
+/* a new chunk's (or a new tuning's) segments: the one-query set now, the
+ * batches' when first used */
+int c2_build_segments(cbp_handle* h, const cbp_profiles* s)
+{
+    h->segs.clear();
     h->chunk_maxlen = 0;
     for (int32_t p = 0; p < s->nprof; p++)
         if (s->len[p] > h->chunk_maxlen) h->chunk_maxlen = s->len[p];
-    for (int32_t i = 0; i < h->nseg; i++) {
-        const int32_t pl = h->seg_p[i + 1] - 1;
-        const int64_t cols = (int64_t)s->dist[pl] + s->len[pl] - (int64_t)s->dist[h->seg_p[i]];
-        if (cols > h->seg_maxcols) h->seg_maxcols = (int32_t)cols;
+    h->segs.emplace_back(new SegSet());
+    return build_segset(h, s, seg_target(h, s->npos, 1), h->segs[0].get());
+}
+
+SegSet* c2_segments(cbp_handle* h, int nq, int* rc)
+{
+    *rc = CBP_OK;
+    const int64_t target = seg_target(h, h->dchunk.npos, nq);
+    for (auto& g : h->segs) if (g->target == target) return g.get();
+    /* batches of many sizes: the oldest set goes, with the graphs that may
+     * hold its addresses */
+    if (h->segs.size() >= 8) {
+        (void)hipStreamSynchronize(h->stream);
+        c2_drop_graphs(h);
+        h->segs.erase(h->segs.begin() + 1);
     }
-    int rc;
-    if ((rc = dupload(h, h->dseg_b, h->seg_p.data(), h->nseg))) return rc;
-    if ((rc = dupload(h, h->dseg_e, h->seg_p.data() + 1, h->nseg))) return rc;
-    HIPCHK(hipStreamSynchronize(h->stream));
-    return CBP_OK;
+    std::unique_ptr<SegSet> g(new SegSet());
+    if ((*rc = build_segset(h, &h->chunk.v, target, g.get()))) return nullptr;
+    h->segs.push_back(std::move(g));
+    return h->segs.back().get();
+}
+
+/* as many waves as the tuning and the LDS allow, but no more than spread the
+ * segments over every CU: 150 segments in workgroups of 8 would keep 19 of
+ * 256 CUs busy with two waves on each SIMD */
+int c2_phase1_waves(const cbp_handle* h, int R, int nstripes, int nseg)
+{
+    int nw = h->nw;
+    while (nw > 1 && (c2_phase1_lds_bytes(R, nw, nstripes) > 160 * 1024 || (int64_t)h->ncu * (nw / 2) >= nseg)) nw >>= 1;
+    return nw;
 }
 
 extern "C" {
@@ -462,7 +519,8 @@ int c2_fill_p1args(cbp_handle* h, DevQuery* dq, P1Args* a)
     a->shift = h->opt.mapaln ? 0.002f : 0.0003f;
     a->ssswgt = h->opt.ssswgt;
     c2_fill_cvs(h, dq, &a->cvs);
-    a->seg_pb = h->dseg_b.as<int32_t>(); a->seg_pe = h->dseg_e.as<int32_t>(); a->nseg = h->nseg;
+    const SegSet& g = *h->segs[0];
+    a->seg_pb = g.db.as<int32_t>(); a->seg_pe = g.de.as<int32_t>(); a->nseg = g.nseg;
     a->mfma = h->use_mfma;
     return CBP_OK;
 }
@@ -549,8 +607,7 @@ int c2_run_phase1(cbp_handle* h, int qidx)
     if ((rc = dalloc(h, h->wts, sizeof(float) * 20 * (size_t)h->dchunk.nprof))) return rc;
     a.wts = h->wts.as<float>();
     HIPCHK(c2_launch_weights(dq->qbkg.as<float>(), h->dchunk.bkg.as<float>(), h->dchunk.nprof, h->wts.as<float>(), h->stream));
-    int nw = h->nw;
-    while (nw > 1 && c2_phase1_lds_bytes(dq->hp.R, nw, dq->hp.nstripes) > 160 * 1024) nw >>= 1;
+    const int nw = c2_phase1_waves(h, dq->hp.R, dq->hp.nstripes, a.nseg);
     HIPCHK(hipMemsetAsync(h->keys.p, 0, sizeof(unsigned long long) * h->dchunk.nprof, h->stream));
     HIPCHK(hipEventRecord(h->ev0, h->stream));
     HIPCHK(c2_launch_phase1(a, dq->hp.R, nw, false, h->stream));

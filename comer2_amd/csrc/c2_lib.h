@@ -186,6 +186,15 @@ struct DlResult {
     std::vector<char> strs;
 };
 
+/* the chunk cut into segments of whole profiles, the unit of work of one
+ * phase-1 wave, widest first */
+struct SegSet {
+    int64_t target = 0;                 /* columns a segment aims at */
+    std::vector<int32_t> b, e;          /* first profile, one past the last */
+    int32_t nseg = 0, maxcols = 0;      /* segments, columns of the widest */
+    DBuf db, de;
+};
+
 constexpr int C2_NSTREAMS = 4;
 constexpr size_t C2_QCACHE_MAX = 128;
 /* one-query calls run the candidates' histograms ahead of the finalize when
@@ -213,8 +222,10 @@ struct cbp_handle {
     HostSet chunk;
     DevSet dchunk;
     bool have_chunk = false;
-    std::vector<int32_t> seg_p;
-    DBuf dseg_b, dseg_e;
+    /* segment sets of the chunk, by target width; the first one is a
+     * one-query launch's */
+    std::vector<std::unique_ptr<SegSet>> segs;
+    int ncu = 256;       /* compute units of the device */
     DBuf dnnw;           /* SS18 parameters on the device */
     /* context-vector map (cbp_upload_cvs2s) and the model's constants */
     std::vector<float> cvkeys, cvvals;
@@ -224,12 +235,11 @@ struct cbp_handle {
     /* per-call scratch */
     DBuf cand, cand_off, btck, fin, pass_pro, counts, statin, statout;
     DBuf mpairs, mF, mSd, mhand, mbt, mstat, malns, malntmp, mres;
-    int32_t nseg = 0;
     DBuf keys;           /* [nprof] u64 */
     DBuf bot;            /* stripe hand-off */
     DBuf wts;            /* [nprof][20] score weights of the query being searched */
     uint64_t dblen = 0, nseqs = 0;
-    int seg_cols = 4096; /* tuning: target columns per segment */
+    int seg_cols = 4096; /* tuning: target columns per segment (narrower for a chunk too small to fill the device) */
     int rmax = 5;        /* tuning: max rows per lane */
     int nw = 8;          /* tuning: waves per workgroup */
     double last_ms = 0.0;
@@ -270,7 +280,6 @@ struct cbp_handle {
     QPlan qscan, qcand;
     DBuf qkeys, qwts;                   /* [nq][nprof] maxima, [nq][nprof][20] weights */
     unsigned long long* hqkeys = nullptr; size_t hqkeys_n = 0;
-    int32_t seg_maxcols = 0;            /* columns of the widest segment */
     hipEvent_t gfork = nullptr, gjoin[C2_NSTREAMS - 1] = {nullptr, nullptr, nullptr};
     hipEvent_t gt0 = nullptr, gt1 = nullptr;
     /* fork/join of the MAP backward pass beside the forward pass (one-query
@@ -339,6 +348,11 @@ constexpr float C2_CV_UNINF = 0.17302947f;
 void c2_fill_scorectx(cbp_handle* h, DevQuery* dq, ScoreCtx* c);
 uint64_t c2_length_adjustment(const cbp_options& o, uint64_t m, uint64_t n, uint64_t N, uint64_t* delta);
 int c2_build_segments(cbp_handle* h, const cbp_profiles* s);
+/* the chunk's segments for nq queries in one launch sequence (built on
+ * first use); null on failure */
+SegSet* c2_segments(cbp_handle* h, int nq, int* rc);
+/* waves per workgroup of a one-query launch over nseg segments */
+int c2_phase1_waves(const cbp_handle* h, int R, int nstripes, int nseg);
 int c2_run_phase1(cbp_handle* h, int qidx);
 int c2_run_queries(cbp_handle* h, const int32_t* qidx, int32_t nq, const float* scorethld,
                    const float* logevthld, cbp_results* outs);

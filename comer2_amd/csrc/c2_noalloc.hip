@@ -107,11 +107,11 @@ extern "C" int cbp_phase1_keys_noalloc(cbp_handle* h, int32_t qidx, uint64_t* ke
     a.Lq = hp.Lq; a.Lpad = hp.Lpad; a.nstripes = hp.nstripes;
     a.shift = h->opt.mapaln ? 0.002f : 0.0003f;
     a.ssswgt = h->opt.ssswgt;
-    a.seg_pb = h->dseg_b.as<int32_t>(); a.seg_pe = h->dseg_e.as<int32_t>(); a.nseg = h->nseg;
+    const SegSet& g = *h->segs[0];
+    a.seg_pb = g.db.as<int32_t>(); a.seg_pe = g.de.as<int32_t>(); a.nseg = g.nseg;
     a.keys = (unsigned long long*)(base + o_keys);
     a.bot = hp.nstripes > 1 ? (float*)(base + o_bot) : nullptr;
-    int nw = h->nw;
-    while (nw > 1 && c2_phase1_lds_bytes(hp.R, nw, hp.nstripes) > 160 * 1024) nw >>= 1;
+    const int nw = c2_phase1_waves(h, hp.R, hp.nstripes, a.nseg);
     /* the maxima start at zero (a kernel, not a memset) */
     if (c2_launch_zero_u64(a.keys, (int64_t)np, st) != hipSuccess ||
         c2_launch_weights(a.qbkg, a.bkg, (int)np, wts, st) != hipSuccess ||

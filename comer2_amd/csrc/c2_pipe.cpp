@@ -74,8 +74,7 @@ int phase1_launch(cbp_handle* h, QWork& w, bool timed, bool copy = true)
     if ((rc = c2_fill_p1args(h, dq, &a))) return rc;
     a.keys = w.dk;
     if (dq->hp.nstripes > 1) a.bot = h->sbot[w.slot].as<float>();
-    int nw = h->nw;
-    while (nw > 1 && c2_phase1_lds_bytes(dq->hp.R, nw, dq->hp.nstripes) > 160 * 1024) nw >>= 1;
+    const int nw = c2_phase1_waves(h, dq->hp.R, dq->hp.nstripes, a.nseg);
     a.wts = w.dw;
     PCHK(c2_launch_zero_u64(w.dk, np, w.st));
     PCHK(c2_launch_weights(dq->qbkg.as<float>(), h->dchunk.bkg.as<float>(), np, w.dw, w.st));
@@ -204,7 +203,12 @@ int queue_scan_prepare(cbp_handle* h, int nq)
     }
     cbp_handle::QPlan& P = h->qscan;
     P.args.resize(nq);
-    P.bot_ld = h->seg_maxcols;
+    const SegSet* sg = c2_segments(h, nq, &rc);
+    if (!sg) return rc;
+    P.bot_ld = sg->maxcols;
+    /* a batch of fewer segments than 4 waves on every CU: smaller workgroups
+     * spread them */
+    const int nwmax = h->nw >= 8 && (int64_t)nq * sg->nseg > (int64_t)4 * h->ncu ? 8 : 4;
     const cbp_profiles& ch = h->chunk.v;
     std::vector<std::vector<QTileCost>> perq(nq);
     std::vector<int> nwq(nq);
@@ -218,15 +222,16 @@ int queue_scan_prepare(cbp_handle* h, int nq)
         if ((rc = c2_fill_p1args(h, w.dq, &P.args[i]))) return rc;
         P.args[i].keys = w.dk;
         P.args[i].wts = w.dw;
-        int nw = h->nw >= 8 ? 8 : 4;
+        P.args[i].seg_pb = sg->db.as<int32_t>(); P.args[i].seg_pe = sg->de.as<int32_t>(); P.args[i].nseg = sg->nseg;
+        int nw = nwmax;
         if (nw == 8 && c2_phase1_lds_bytes(hp.R, 8, hp.nstripes) > 160 * 1024) nw = 4;
         nwq[i] = nw;
-        const int ng = (h->nseg + nw - 1) / nw;
+        const int ng = (sg->nseg + nw - 1) / nw;
         perq[i].resize(ng);
         for (int g = 0; g < ng; g++) {
-            const int s0 = g * nw, s1 = std::min(h->nseg, s0 + nw);
-            const int32_t pb = h->seg_p[s0], pl = h->seg_p[s1] - 1;
-            const double cols = (double)((int64_t)ch.dist[pl] + ch.len[pl] - (int64_t)ch.dist[pb]) / (s1 - s0);
+            /* widest first: the group lasts as long as its first segment */
+            const int32_t pb = sg->b[g * nw], pl = sg->e[g * nw] - 1;
+            const double cols = (double)((int64_t)ch.dist[pl] + ch.len[pl] - (int64_t)ch.dist[pb]);
             perq[i][g] = QTileCost{(double)hp.nstripes * hp.R * (cols + 63.0), i, g};
         }
     }

@@ -1,0 +1,54 @@
+"""Phase-1 segments and waves per workgroup chosen from the chunk's size: the
+maxima equal the oracle's at the counts where the launch shape changes, for
+databases in any order, and a batch's queue equals the one-query launches."""
+import numpy as np
+import pytest
+from comer2_amd._ffi import SynthDB
+from gpu_common import expected_keys, oracle, processing
+
+pytestmark = pytest.mark.gpu
+
+
+# 1, 2, 4 and 8 waves per workgroup start at 1, 257, 513 and 1,025 segments
+# (one profile each here), on both sides of each line; one and two stripes
+@pytest.mark.parametrize("nprof,qlen", [(n, 37) for n in (1, 3, 256, 257, 512, 513, 1024, 1025)] +
+                         [(n, 333) for n in (1, 3, 257, 513, 1025)])
+def test_segment_counts(nprof, qlen):
+    rng = np.random.default_rng(nprof)
+    lens = rng.integers(30, 44, nprof)
+    q = SynthDB.from_lengths(201, [qlen])
+    d = SynthDB.from_lengths(202, lens)
+    print(f"segments: {nprof} profiles, query {qlen}", flush=True)
+    cbp = processing()
+    cbp.TransferQueries(q)
+    cbp.TransferCPMData(d)
+    assert np.array_equal(cbp.phase1_keys(0), expected_keys(oracle(), q, 0, d))
+
+
+@pytest.mark.parametrize("order", ["longest", "shortest", "mixed"])
+def test_segment_order_and_batches(order):
+    rng = np.random.default_rng(5)
+    lens = np.sort(np.clip(np.rint(120 * np.exp(0.668 * rng.standard_normal(700))), 30, 900).astype(np.int32))
+    lens = {"longest": lens[::-1], "shortest": lens, "mixed": rng.permutation(lens)}[order]
+    q = SynthDB.from_lengths(211, [64, 65, 330])
+    d = SynthDB.from_lengths(212, lens)
+    d.plant(q, 213, 20, 3.0, 60.0)
+    cbp = processing(dict(max_map_pairs=8))
+    cbp.TransferQueries(q)
+    cbp.TransferCPMData(d)
+    cbp.SetDbDetails(d.npos, d.nprof)
+    print(f"segment order {order}", flush=True)
+    one = [cbp.ProcessScoreMatrix(i) for i in range(3)]
+    for qs in ([0, 1, 2], [0, 2], [0, 1, 2] * 6):
+        for i, r in zip(qs, cbp.ProcessBatch(qs)):
+            assert np.array_equal(r["alndata"].view(np.uint32), one[i]["alndata"].view(np.uint32)), (order, qs, i)
+            assert np.array_equal(r["order"], one[i]["order"])
+            assert np.array_equal(r["aln_raw"], one[i]["aln_raw"])
+    keys = cbp.phase1_keys(2)
+    pick = np.linspace(0, d.nprof - 1, 40).astype(int)
+    orc = oracle()
+    from comer2_amd.host import encode_key
+    for dp in pick:
+        S, _ = orc.score_f32(q.view, 2, d.view, int(dp))
+        m, _, _ = orc.viterbi_f32(q.view, 2, d.view, int(dp), S)
+        assert int(keys[dp]) == encode_key(m.maxsc, m.x, m.y), (order, dp)
