@@ -883,7 +883,7 @@ extern "C" int cbp_sdp_forward(cbp_handle* h, const float* S, const float* theta
     SdpArgs a;
     sdp_fill(h, &a, S, theta, ws);
     a.logZ = logZ;
-    HIPCHK(c2_launch_sdp(a, false, h->sdp_groups, h->sdp_nw, stream ? (hipStream_t)stream : h->stream));
+    HIPCHK(c2_launch_sdp(a, false, h->sdp_groups, h->sdp_nw, (hipStream_t)stream));
     return CBP_OK;
 }
 
@@ -897,7 +897,7 @@ extern "C" int cbp_sdp_adjoint(cbp_handle* h, const float* S, const float* theta
     SdpArgs a;
     sdp_fill(h, &a, S, theta, ws);
     a.logZ = (float*)logZ; a.gZ = gZ; a.dS = dS; a.dth = dtheta; a.post = post;
-    HIPCHK(c2_launch_sdp(a, true, h->sdp_groups, h->sdp_nw, stream ? (hipStream_t)stream : h->stream));
+    HIPCHK(c2_launch_sdp(a, true, h->sdp_groups, h->sdp_nw, (hipStream_t)stream));
     return CBP_OK;
 }
 
@@ -919,7 +919,7 @@ extern "C" int cbp_sdp_scores(cbp_handle* h, float* S, void* stream)
     a.shift = h->opt.mapaln ? 0.002f : 0.0003f;
     a.ssswgt = h->opt.ssswgt;
     a.S = S;
-    HIPCHK(c2_launch_sdp_scores(a, (int)h->sdp_pairs.size(), stream ? (hipStream_t)stream : h->stream));
+    HIPCHK(c2_launch_sdp_scores(a, (int)h->sdp_pairs.size(), (hipStream_t)stream));
     return CBP_OK;
 }
 

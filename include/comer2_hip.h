@@ -440,7 +440,8 @@ int  cbp_last_kernel_ms(const cbp_handle* h, double* ms, int32_t* nlaunch);
  * dlogZ/dS, dlogZ/dtheta and, optionally, the MM posteriors
  * exp(F+B-logZ), the quantity of CuBatchMAPDP_bwd.cu:531-544.
  * S, theta, logZ, gZ, dS, dtheta, post and ws are device pointers; stream is
- * a hipStream_t (NULL: the handle's stream); calls are asynchronous. */
+ * a hipStream_t (NULL: the default stream, which waits for the handle's own
+ * stream and is waited for by it); calls are asynchronous. */
 typedef struct {
     int32_t qidx;        /* query index in the uploaded query set */
     int32_t pronr;       /* profile index in the uploaded chunk */
