@@ -271,14 +271,15 @@ int64_t c2_sdp_ckpt_floats(int R);
 /* groups persistent workgroups of nw waves (one stripe each) */
 hipError_t c2_launch_sdp(const SdpArgs& a, bool adjoint, int groups, int nw, hipStream_t stream);
 struct SdpScoreArgs {
-    const SdpPair* pairs;
+    const SdpPair* pairs; const int2* items;   /* items: (pair, first query row) */
     const float* qtrg; const float* qss; const float* qbkg; const uint32_t* qdist; int64_t qnpos; int32_t qnprof;
     const float* dtrg; const float* dss; const float* dbkg; const uint32_t* ddist; int64_t dnpos; int32_t dnprof;
     const float* ssss;   /* [30][30] */
     float shift, ssswgt;
     float* S;
 };
-hipError_t c2_launch_sdp_scores(const SdpScoreArgs& a, int npairs, hipStream_t stream);
+int c2_sdp_score_rows();    /* query rows of an item */
+hipError_t c2_launch_sdp_scores(const SdpScoreArgs& a, int nitems, hipStream_t stream);
 /* S and mod of query vs chunk profile p (Ld its length), row-major [Lq][Ld] */
 hipError_t c2_launch_score_block(const ScoreCtx& c, int p, int Ld, float* S, float* mod, hipStream_t stream);
 

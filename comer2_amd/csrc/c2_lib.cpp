@@ -853,6 +853,12 @@ extern "C" int cbp_sdp_prepare(cbp_handle* h, const cbp_sdp_pair* pairs, int32_t
         if ((rc = dupload(h, h->sdp_dpairs, h->sdp_pairs.data(), h->sdp_pairs.size()))) return rc;
         if ((rc = dupload(h, h->sdp_dorder, h->sdp_order.data(), h->sdp_order.size()))) return rc;
     }
+    std::vector<int2> items;
+    for (int32_t i = 0; i < npairs; i++)
+        for (int32_t r = 0; r < h->sdp_pairs[i].L1; r += c2_sdp_score_rows()) items.push_back(make_int2(i, r));
+    if (items.size() > (size_t)0x7fffffff) return fail(h, CBP_ERR_ARG, "soft DP: too many pairs");
+    h->sdp_nitems = (int32_t)items.size();
+    if (npairs > 0 && (rc = dupload(h, h->sdp_ditems, items.data(), items.size()))) return rc;
     HIPCHK(hipStreamSynchronize(h->stream));
     *ws_bytes = off * (int64_t)sizeof(float);
     h->sdp_ready = true;
@@ -910,7 +916,7 @@ extern "C" int cbp_sdp_scores(cbp_handle* h, float* S, void* stream)
     (void)hipSetDevice(h->device);
     const cbp_profiles& q = h->queries.v;
     SdpScoreArgs a;
-    a.pairs = h->sdp_dpairs.as<SdpPair>();
+    a.pairs = h->sdp_dpairs.as<SdpPair>(); a.items = h->sdp_ditems.as<int2>();
     a.qtrg = h->sdq_trg.as<float>(); a.qss = h->sdq_ss.as<float>(); a.qbkg = h->sdq_bkg.as<float>();
     a.qdist = h->sdq_dist.as<uint32_t>(); a.qnpos = q.npos; a.qnprof = q.nprof;
     a.dtrg = h->dchunk.trgfrq.as<float>(); a.dss = h->dchunk.ssprb.as<float>(); a.dbkg = h->dchunk.bkg.as<float>();
@@ -919,7 +925,7 @@ extern "C" int cbp_sdp_scores(cbp_handle* h, float* S, void* stream)
     a.shift = h->opt.mapaln ? 0.002f : 0.0003f;
     a.ssswgt = h->opt.ssswgt;
     a.S = S;
-    HIPCHK(c2_launch_sdp_scores(a, (int)h->sdp_pairs.size(), (hipStream_t)stream));
+    HIPCHK(c2_launch_sdp_scores(a, h->sdp_nitems, (hipStream_t)stream));
     return CBP_OK;
 }
 

@@ -311,7 +311,8 @@ struct cbp_handle {
     bool sdq_ready = false;
     std::vector<SdpPair> sdp_pairs;
     std::vector<int32_t> sdp_order;
-    DBuf sdp_dpairs, sdp_dorder;
+    DBuf sdp_dpairs, sdp_dorder, sdp_ditems;
+    int32_t sdp_nitems = 0;      /* score items (pair, rows) */
     int32_t sdp_K = 0, sdp_nw = 1, sdp_groups = 1;
     int64_t sdp_ws_floats = 0, sdp_scr_off = 0;
     bool sdp_ready = false;

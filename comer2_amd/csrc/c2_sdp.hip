@@ -690,40 +690,108 @@ __global__ __launch_bounds__(512) void k_sdp_adj(SdpArgs a)
 
 /* score matrices of the prepared pairs from the raw profile fields:
  * S = log(sum_a q_a d_a / (0.5 (bq_a + bd_a))) - shift
- *     + ssswgt (sum_st p_s p'_t T[10s+int(9.999 p_s)][10t+int(9.999 p'_t)]
- *               + (p_H+0.1)(p'_H+0.1) 0.1111111 - 0.05)
- * (CalcSM_Init_SMEMUnroll2x + CalcSM_SSSS_SMEMUnroll2x); one workgroup per pair */
+ *     + ssswgt (sum_j p'_j QT[10j+int(9.999 p'_j)] + (p_H+0.1)(p'_H+0.1) 0.1111111 - 0.05),
+ * QT(row)[g] = sum_i p_i T[10i+int(9.999 p_i)][g]
+ * (CalcSM_Init_SMEMUnroll2x + CalcSM_SSSS_SMEMUnroll2x), the operations of
+ * the search kernels.
+ *
+ * One workgroup per item of (pair, SC_ROWS query rows): the rows'
+ * frequencies and SS tables go to LDS, and the waves take units of 16 rows x
+ * 64 columns, a column's 20 weighted frequencies in a lane's registers, four
+ * rows at a time (16-byte LDS reads); a row's 64 scores are one 256-byte
+ * store.  Bound by VALU issue (about 55 operations a cell).  1,024 pairs of
+ * 50-600 (108 M cells): 1.19 -> 0.25 ms (430 GCUPS); one workgroup per
+ * pair re-read both profiles' 23 fields from memory for every cell.  Rows in
+ * scalar registers (four or two at a time) spilled them and ran 0.36-0.40. */
+constexpr int SC_ROWS = 32;
+
 __global__ __launch_bounds__(256) void k_sdp_scores(SdpScoreArgs a)
 {
-    __shared__ float T[900];
+    __shared__ __align__(16) float qt[30][SC_ROWS], qf[20][SC_ROWS];
+    __shared__ __align__(16) float qh[SC_ROWS];
     __shared__ float w[20];
-    for (int i = threadIdx.x; i < 900; i += blockDim.x) T[i] = a.ssss[i];
-    const SdpPair P = a.pairs[blockIdx.x];
-    if (threadIdx.x < 20)
-        w[threadIdx.x] = 1.0f / (0.5f * (a.qbkg[(size_t)threadIdx.x * a.qnprof + P.q] +
-                                         a.dbkg[(size_t)threadIdx.x * a.dnprof + P.p]));
-    __syncthreads();
-    const int64_t q0 = a.qdist[P.q], d0 = a.ddist[P.p];
-    const int64_t n = (int64_t)P.L1 * P.L2;
-    for (int64_t i = threadIdx.x; i < n; i += blockDim.x) {
-        const int r = (int)(i / P.L2), c = (int)(i - (int64_t)r * P.L2);
-        float acc = 0.0f;
-        for (int k = 0; k < 20; k++)
-            acc = fmaf(a.qtrg[(size_t)k * a.qnpos + q0 + r], a.dtrg[(size_t)k * a.dnpos + d0 + c] * w[k], acc);
-        float sc = c2_logf_clamped(acc) - a.shift;
-        if (a.ssswgt > 0.0f) {
-            float ps[3], pt[3]; int is[3], it[3];
-            for (int j = 0; j < 3; j++) {
-                ps[j] = a.qss[(size_t)j * a.qnpos + q0 + r]; is[j] = 10 * j + (int)(ps[j] * 9.999f);
-                pt[j] = a.dss[(size_t)j * a.dnpos + d0 + c]; it[j] = 10 * j + (int)(pt[j] * 9.999f);
-            }
-            float ss = 0.0f;
-            for (int x = 0; x < 3; x++)
-                for (int y = 0; y < 3; y++) ss = fmaf(ps[x] * pt[y], T[is[x] * 30 + it[y]], ss);
-            ss = fmaf(ps[2] + 0.1f, (pt[2] + 0.1f) * 0.1111111f, ss);
-            sc += (ss - 0.05f) * a.ssswgt;
+    const int pi = __builtin_amdgcn_readfirstlane(a.items[blockIdx.x].x);
+    const int r0 = __builtin_amdgcn_readfirstlane(a.items[blockIdx.x].y);
+    const SdpPair P = a.pairs[pi];
+    const int nr = min(SC_ROWS, P.L1 - r0);
+    const int64_t q0 = (int64_t)a.qdist[P.q] + r0, d0 = a.ddist[P.p];
+    const bool ss_on = a.ssswgt > 0.0f;
+    if (ss_on) {
+        for (int i = threadIdx.x; i < 30 * SC_ROWS; i += blockDim.x) {
+            const int g = i / SC_ROWS, r = i % SC_ROWS;
+            float v = 0.0f;
+            if (r < nr) {
+                const float p0 = a.qss[q0 + r], p1 = a.qss[(size_t)a.qnpos + q0 + r], p2 = a.qss[2 * (size_t)a.qnpos + q0 + r];
+                v = p0 * a.ssss[(int)(p0 * 9.999f) * 30 + g];
+                v = fmaf(p1, a.ssss[(10 + (int)(p1 * 9.999f)) * 30 + g], v);
+                v = fmaf(p2, a.ssss[(20 + (int)(p2 * 9.999f)) * 30 + g], v);
+                if (g == 0) qh[r] = p2 + 0.1f;
+            } else if (g == 0) qh[r] = 0.0f;
+            qt[g][r] = v;
         }
-        a.S[P.soff + i] = sc;
+    }
+    for (int i = threadIdx.x; i < 20 * SC_ROWS; i += blockDim.x) {
+        const int k = i / SC_ROWS, r = i % SC_ROWS;
+        qf[k][r] = r < nr ? a.qtrg[(size_t)k * a.qnpos + q0 + r] : 0.0f;
+    }
+    if (threadIdx.x < 20)
+        w[threadIdx.x] = 1.0f / (0.5f * (a.qbkg[(size_t)threadIdx.x * a.qnprof + P.q] + a.dbkg[(size_t)threadIdx.x * a.dnprof + P.p]));
+    __syncthreads();
+    const int lane = threadIdx.x & 63;
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    float* out = a.S + P.soff + (int64_t)r0 * P.L2;
+    /* units of 16 rows x 64 columns, dealt to the waves */
+    const int nblk = (P.L2 + 63) / 64, nun = nblk * ((nr + 15) / 16);
+    for (int u = wv; u < nun; u += 4) {
+        const int half = u >= nblk ? 1 : 0;
+        const int c = 64 * (u - half * nblk) + lane;
+        const bool ok = c < P.L2;
+        const int64_t col = d0 + (ok ? c : 0);
+        float dw[20], pj[3], dh = 0.0f;
+        int it[3] = {0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < 20; k++) dw[k] = a.dtrg[(size_t)k * a.dnpos + col] * w[k];
+        if (ss_on) {
+#pragma unroll
+            for (int j = 0; j < 3; j++) {
+                pj[j] = a.dss[(size_t)j * a.dnpos + col];
+                it[j] = 10 * j + (int)(pj[j] * 9.999f);
+            }
+            dh = (pj[2] + 0.1f) * 0.1111111f;
+        }
+        const int re = min(nr, 16 * half + 16);
+        for (int r = 16 * half; r < re; r += 4) {
+            float acc[4] = {0.0f, 0.0f, 0.0f, 0.0f}, sc[4];
+#pragma unroll
+            for (int k = 0; k < 20; k++) {
+                const float4 q = *(const float4*)&qf[k][r];
+                acc[0] = fmaf(q.x, dw[k], acc[0]); acc[1] = fmaf(q.y, dw[k], acc[1]);
+                acc[2] = fmaf(q.z, dw[k], acc[2]); acc[3] = fmaf(q.w, dw[k], acc[3]);
+            }
+            c2_logf_clamped_n<4>(acc, sc);
+#pragma unroll
+            for (int n = 0; n < 4; n++) sc[n] = sc[n] - a.shift;
+            if (ss_on) {
+                const float4 t0 = *(const float4*)&qt[it[0]][r], t1 = *(const float4*)&qt[it[1]][r],
+                             t2 = *(const float4*)&qt[it[2]][r], h4 = *(const float4*)&qh[r];
+                const float x0[4] = {t0.x, t0.y, t0.z, t0.w}, x1[4] = {t1.x, t1.y, t1.z, t1.w},
+                            x2[4] = {t2.x, t2.y, t2.z, t2.w}, xh[4] = {h4.x, h4.y, h4.z, h4.w};
+#pragma unroll
+                for (int n = 0; n < 4; n++) {
+                    float ss = x0[n] * pj[0];
+                    ss = fmaf(x1[n], pj[1], ss);
+                    ss = fmaf(x2[n], pj[2], ss);
+                    ss = fmaf(xh[n], dh, ss);
+                    sc[n] += (ss - 0.05f) * a.ssswgt;
+                }
+            }
+            if (ok) {
+                float* o = out + (int64_t)r * P.L2 + c;
+#pragma unroll
+                for (int n = 0; n < 4; n++)
+                    if (r + n < re) o[(int64_t)n * P.L2] = sc[n];
+            }
+        }
     }
 }
 
@@ -754,10 +822,12 @@ hipError_t c2_launch_sdp(const SdpArgs& a, bool adjoint, int groups, int nw, hip
     return hipGetLastError();
 }
 
-hipError_t c2_launch_sdp_scores(const SdpScoreArgs& a, int npairs, hipStream_t stream)
+int c2_sdp_score_rows() { return SC_ROWS; }
+
+hipError_t c2_launch_sdp_scores(const SdpScoreArgs& a, int nitems, hipStream_t stream)
 {
     (void)hipGetLastError();   /* the status read after the launches is theirs alone */
-    if (npairs <= 0) return hipSuccess;
-    hipLaunchKernelGGL(k_sdp_scores, dim3(npairs), dim3(256), 0, stream, a);
+    if (nitems <= 0) return hipSuccess;
+    hipLaunchKernelGGL(k_sdp_scores, dim3(nitems), dim3(256), 0, stream, a);
     return hipGetLastError();
 }
