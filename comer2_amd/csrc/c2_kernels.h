@@ -245,17 +245,24 @@ int c2_phase1q_grid(int R, int NW, bool btck, size_t lds, bool mf = false);
 hipError_t c2_launch_phase1q(const P1QueueArgs& q, int R, int NW, bool btck, int grid, size_t lds, hipStream_t stream,
                              bool mf = false);
 
+constexpr int C2_SDP_BAND = 4;      /* waves of a soft-DP workgroup, one stripe each */
 /* soft DP: one pair of (query, chunk profile) and its workspace offsets (floats) */
 struct SdpPair {
     int32_t q, p;        /* query index, chunk profile index */
     int32_t L1, L2;      /* lengths */
-    int32_t ns, ncp;     /* stripes of 64*R rows; checkpoint slots per stripe */
+    int32_t ns, ncp;     /* stripes of 64 rows; checkpoint slots per stripe */
+    int32_t nb, i0;      /* bands of up to C2_SDP_BAND stripes; bands of the pairs before */
     int64_t soff;        /* offset of the pair's [L1][L2] block in S / dS / posterior */
     int64_t foff;        /* forward store: all cells (K = 0) or checkpoints */
-    int64_t hoff;        /* stripe hand-offs: forward [ns][5][L2], then adjoint [3][L2] */
+    int64_t hoff;        /* with checkpoints, the stripes' last rows [ns][5][L2] */
+    int64_t boff;        /* the bands' last rows but the last [nb-1][5][L2] (forward) */
+    int64_t aoff;        /* the bands' first rows [nb][3][L2] (adjoint) */
 };
 struct SdpArgs {
-    const SdpPair* pairs; const int32_t* order; int32_t npairs;
+    const SdpPair* pairs; int32_t npairs;
+    const int2* items; int32_t nitems;                       /* (pair, band): longest pairs first, a pair's
+                                                                bands in the order of the sweep */
+    unsigned* head;                                          /* item counter (null: one band per pair) */
     const float* qtr; int64_t qntr; const uint32_t* qdist;   /* query set transitions [7][npos+nprof] */
     const float* qll; const float* qld;                      /* column -1 vectors [qnpos][5] */
     const float* dtr; int64_t dntr; const uint32_t* ddist;   /* chunk transitions */
@@ -264,12 +271,14 @@ struct SdpArgs {
     float* dS; float* dth; float* post;                      /* adjoint outputs */
     float* ws;                                               /* workspace */
     int64_t scr_off;                                         /* per-wave segment scratch */
+    int64_t zpart_off, dpart_off;                            /* the bands' sums: [items][2] f32, [items][5] f64 */
     int32_t K;                                               /* checkpoint interval (divides 64), 0 = store all */
 };
-int c2_sdp_rows_per_lane();
-int64_t c2_sdp_ckpt_floats(int R);
-/* groups persistent workgroups of nw waves (one stripe each) */
-hipError_t c2_launch_sdp(const SdpArgs& a, bool adjoint, int groups, int nw, hipStream_t stream);
+int64_t c2_sdp_ckpt_floats();       /* a stripe's checkpoint */
+int64_t c2_sdp_group_floats();      /* a stripe's four stored steps */
+/* groups persistent workgroups of nw waves (one stripe each); xoff, xn: the
+ * pass's hand-off rows between bands in the workspace */
+hipError_t c2_launch_sdp(const SdpArgs& a, bool adjoint, int groups, int nw, int64_t xoff, int64_t xn, hipStream_t stream);
 struct SdpScoreArgs {
     const SdpPair* pairs; const int2* items;   /* items: (pair, first query row) */
     const float* qtrg; const float* qss; const float* qbkg; const uint32_t* qdist; int64_t qnpos; int32_t qnprof;

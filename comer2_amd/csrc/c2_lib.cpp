@@ -796,7 +796,6 @@ extern "C" int cbp_sdp_prepare(cbp_handle* h, const cbp_sdp_pair* pairs, int32_t
     h->sdp_ready = false;
     int rc;
     if ((rc = sdp_upload_queries(h))) return rc;
-    const int R = c2_sdp_rows_per_lane();
     const cbp_profiles& q = h->queries.v;
     const cbp_profiles& d = h->chunk.v;
     int maxsteps = 1;
@@ -813,45 +812,73 @@ extern "C" int cbp_sdp_prepare(cbp_handle* h, const cbp_sdp_pair* pairs, int32_t
     if (K < 0) K = (int)std::ceil(std::sqrt((double)maxsteps));
     if (K > 0) K = K >= 64 ? 64 : (K >= 32 ? 32 : 16);
     const auto align = [](int64_t x) { return (x + 63) & ~(int64_t)63; };
+    /* a workgroup's band: a pair's stripes, at most 4: two workgroups then
+     * fit a CU with the adjoint's registers, and a pair of few stripes leaves
+     * few wave slots idle (1,024 pairs of 50-600, a step: bands of 8 4.93 ms,
+     * 4 4.03; 24 pairs of 2,000-5,000 25.8 and 21.5) */
+    int maxL1 = 1;
+    for (int32_t i = 0; i < npairs; i++) maxL1 = std::max(maxL1, (int)q.len[pairs[i].qidx]);
+    const int nw = std::min(C2_SDP_BAND, (maxL1 + 63) / 64);
     h->sdp_pairs.resize(npairs);
-    int64_t off = 0;
+    int64_t off = 0, nbands = 0;
     for (int32_t i = 0; i < npairs; i++) {
         SdpPair& P = h->sdp_pairs[i];
         P.q = pairs[i].qidx; P.p = pairs[i].pronr;
         P.L1 = q.len[P.q]; P.L2 = d.len[P.p];
-        P.ns = (P.L1 + 64 * R - 1) / (64 * R);
+        P.ns = (P.L1 + 63) / 64;
+        P.nb = (P.ns + nw - 1) / nw;
+        P.i0 = (int32_t)nbands;
+        nbands += P.nb;
         const int nsteps = P.L2 + 63;
         P.ncp = K > 0 ? (nsteps - 1) / K + 1 : 0;
         P.soff = pairs[i].soff;
         P.foff = off;
-        off += align(K > 0 ? (int64_t)P.ns * P.ncp * c2_sdp_ckpt_floats(R)
-                           : (int64_t)P.ns * nsteps * 5 * R * 64);
+        off += align(K > 0 ? (int64_t)P.ns * P.ncp * c2_sdp_ckpt_floats()
+                           : (int64_t)P.ns * ((nsteps + 3) / 4) * c2_sdp_group_floats());
         P.hoff = off;
-        off += align((int64_t)P.ns * 5 * P.L2 + 3 * (int64_t)P.L2);
+        if (K > 0) off += align((int64_t)P.ns * 5 * P.L2);
     }
-    /* longest first (cost = stripes x steps), ties by pair index */
-    h->sdp_order.resize(npairs);
-    for (int32_t i = 0; i < npairs; i++) h->sdp_order[i] = i;
-    std::stable_sort(h->sdp_order.begin(), h->sdp_order.end(), [&](int a, int b) {
+    if (nbands > 0x7fffffff) return fail(h, CBP_ERR_ARG, "soft DP: too many pairs");
+    for (int x = 0; x < 2; x++) {
+        h->sdp_xoff[x] = off;
+        for (SdpPair& P : h->sdp_pairs) {
+            (x == 0 ? P.boff : P.aoff) = off;
+            off += x == 0 ? (int64_t)(P.nb - 1) * 5 * P.L2 : (int64_t)P.nb * 3 * P.L2;
+        }
+        h->sdp_xn[x] = off - h->sdp_xoff[x];
+        off = align(off);
+    }
+    h->sdp_multi = nbands > npairs;
+    h->sdp_head_off = off; off += 64;
+    h->sdp_zoff = off; off += align(2 * nbands);
+    h->sdp_doff = off; off += align(10 * nbands);
+    /* longest first (cost = stripes x steps), ties by pair index; a pair's
+     * bands follow each other in the order of the sweep */
+    std::vector<int32_t> order(npairs);
+    for (int32_t i = 0; i < npairs; i++) order[i] = i;
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
         const SdpPair& A = h->sdp_pairs[a]; const SdpPair& B = h->sdp_pairs[b];
         return (int64_t)A.ns * (A.L2 + 63) > (int64_t)B.ns * (B.L2 + 63);
     });
-    /* workgroups of up to 8 waves (one stripe each), about 4096 waves in
-     * all: a stripe per wave only when the pairs alone do not fill the chip */
-    int maxns = 1;
-    for (const SdpPair& P : h->sdp_pairs) maxns = std::max(maxns, P.ns);
-    const int want = npairs > 0 ? (4096 + npairs - 1) / npairs : 1;
-    const int nw = std::max(1, std::min(std::min(maxns, 8), want));
-    const int groups = std::max(1, std::min(npairs, 4096 / nw));
+    std::vector<int2> bands[2];
+    for (int32_t i : order)
+        for (int b = 0; b < h->sdp_pairs[i].nb; b++) {
+            bands[0].push_back(make_int2(i, b));
+            bands[1].push_back(make_int2(i, h->sdp_pairs[i].nb - 1 - b));
+        }
+    /* about 4096 waves at most: later items go to the workgroups that finish */
+    const int groups = (int)std::max<int64_t>(1, std::min<int64_t>(nbands, 4096 / nw));
     h->sdp_nw = nw;
     h->sdp_groups = groups;
+    h->sdp_nbands = (int32_t)nbands;
     h->sdp_scr_off = off;
-    if (K > 0) off += align((int64_t)groups * nw * K * 5 * R * 64);
+    if (K > 0) off += align((int64_t)groups * nw * (K / 4) * c2_sdp_group_floats());
     h->sdp_K = K;
     h->sdp_ws_floats = off;
     if (npairs > 0) {
         if ((rc = dupload(h, h->sdp_dpairs, h->sdp_pairs.data(), h->sdp_pairs.size()))) return rc;
-        if ((rc = dupload(h, h->sdp_dorder, h->sdp_order.data(), h->sdp_order.size()))) return rc;
+        for (int x = 0; x < 2; x++)
+            if ((rc = dupload(h, h->sdp_dband[x], bands[x].data(), bands[x].size()))) return rc;
     }
     std::vector<int2> items;
     for (int32_t i = 0; i < npairs; i++)
@@ -865,10 +892,13 @@ extern "C" int cbp_sdp_prepare(cbp_handle* h, const cbp_sdp_pair* pairs, int32_t
     return CBP_OK;
 }
 
-static void sdp_fill(cbp_handle* h, SdpArgs* a, const float* S, const float* theta, void* ws)
+static void sdp_fill(cbp_handle* h, SdpArgs* a, const float* S, const float* theta, void* ws, bool adjoint)
 {
     std::memset(a, 0, sizeof *a);
-    a->pairs = h->sdp_dpairs.as<SdpPair>(); a->order = h->sdp_dorder.as<int32_t>();
+    a->pairs = h->sdp_dpairs.as<SdpPair>();
+    a->items = h->sdp_dband[adjoint ? 1 : 0].as<int2>(); a->nitems = h->sdp_nbands;
+    a->head = h->sdp_multi ? (unsigned*)((float*)ws + h->sdp_head_off) : nullptr;
+    a->zpart_off = h->sdp_zoff; a->dpart_off = h->sdp_doff;
     a->npairs = (int32_t)h->sdp_pairs.size();
     const cbp_profiles& q = h->queries.v;
     a->qtr = h->sdq_trans.as<float>(); a->qntr = q.npos + q.nprof; a->qdist = h->sdq_dist.as<uint32_t>();
@@ -887,9 +917,10 @@ extern "C" int cbp_sdp_forward(cbp_handle* h, const float* S, const float* theta
     if (!h->sdp_ready) return fail(h, CBP_ERR_STATE, "soft DP: cbp_sdp_prepare first");
     (void)hipSetDevice(h->device);
     SdpArgs a;
-    sdp_fill(h, &a, S, theta, ws);
+    sdp_fill(h, &a, S, theta, ws, false);
     a.logZ = logZ;
-    HIPCHK(c2_launch_sdp(a, false, h->sdp_groups, h->sdp_nw, (hipStream_t)stream));
+    HIPCHK(c2_launch_sdp(a, false, h->sdp_groups, h->sdp_nw, h->sdp_xoff[0], h->sdp_xn[0],
+                         (hipStream_t)stream));
     return CBP_OK;
 }
 
@@ -901,9 +932,10 @@ extern "C" int cbp_sdp_adjoint(cbp_handle* h, const float* S, const float* theta
     if (!h->sdp_ready) return fail(h, CBP_ERR_STATE, "soft DP: cbp_sdp_prepare first");
     (void)hipSetDevice(h->device);
     SdpArgs a;
-    sdp_fill(h, &a, S, theta, ws);
+    sdp_fill(h, &a, S, theta, ws, true);
     a.logZ = (float*)logZ; a.gZ = gZ; a.dS = dS; a.dth = dtheta; a.post = post;
-    HIPCHK(c2_launch_sdp(a, true, h->sdp_groups, h->sdp_nw, (hipStream_t)stream));
+    HIPCHK(c2_launch_sdp(a, true, h->sdp_groups, h->sdp_nw, h->sdp_xoff[1], h->sdp_xn[1],
+                         (hipStream_t)stream));
     return CBP_OK;
 }
 

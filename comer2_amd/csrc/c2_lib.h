@@ -310,9 +310,13 @@ struct cbp_handle {
     DBuf sdq_trans, sdq_dist, sdq_ll, sdq_ld, sdq_trg, sdq_ss, sdq_bkg, dssss;
     bool sdq_ready = false;
     std::vector<SdpPair> sdp_pairs;
-    std::vector<int32_t> sdp_order;
-    DBuf sdp_dpairs, sdp_dorder, sdp_ditems;
+    DBuf sdp_dpairs, sdp_ditems, sdp_dband[2];
     int32_t sdp_nitems = 0;      /* score items (pair, rows) */
+    /* DP items (pair, band), forward and adjoint order; the hand-off rows
+     * between bands; more than one band in some pair */
+    int32_t sdp_nbands = 0;
+    int64_t sdp_xoff[2] = {0, 0}, sdp_xn[2] = {0, 0}, sdp_head_off = 0, sdp_zoff = 0, sdp_doff = 0;
+    bool sdp_multi = false;
     int32_t sdp_K = 0, sdp_nw = 1, sdp_groups = 1;
     int64_t sdp_ws_floats = 0, sdp_scr_off = 0;
     bool sdp_ready = false;
