@@ -51,19 +51,22 @@ DlCaps dl_caps(cbp_handle* h, const std::vector<int>& lq, const std::vector<int>
     k.capW = std::max<int64_t>(64, std::min<int64_t>(h->dl_capW, allw));
     c2_map_geometry(Lmax, &k.mR, &k.mns, &k.mnw);
     const int64_t chunks = (maxlen + C2_MAP_SCORE_COLS - 1) / C2_MAP_SCORE_COLS;
-    k.capItems = (int64_t)k.capM * 8 * chunks;
     int64_t cells = 0, hand = 0;
+    int nsmax = 1;
     for (int L : lq) {
         int R = 1, ns = 1, nw = 1;
         c2_map_geometry(L, &R, &ns, &nw);
+        nsmax = std::max(nsmax, ns);
         cells = std::max(cells, c2_map_cells(R, ns, maxlen));
         hand = std::max(hand, (c2_map_hand(ns, maxlen) + 63) & ~(int64_t)63);
         if (h->map_rmax2 > 0) {
             c2_map_geometry_short(L, h->map_rmax2, &R, &ns, &nw);
+            nsmax = std::max(nsmax, ns);
             cells = std::max(cells, c2_map_cells(R, ns, maxlen));
             hand = std::max(hand, (c2_map_hand(ns, maxlen) + 63) & ~(int64_t)63);
         }
     }
+    k.capItems = (int64_t)k.capM * nsmax * chunks;
     k.capCells = std::min<int64_t>(h->dl_capCells, (int64_t)k.capM * cells);
     k.capHand = std::min<int64_t>((int64_t)1 << 26, (int64_t)k.capM * hand);
     k.stride = (int64_t)Lmax + maxlen + 1;

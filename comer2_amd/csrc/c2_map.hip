@@ -30,6 +30,7 @@
  * cucom/myfastapproxmath.cuh), so results match it bit for bit whatever the
  * schedule; log Z is summed in the reference's block order.
  */
+#include <type_traits>
 #include "c2_draw.h"
 
 namespace {
@@ -425,23 +426,91 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(R == 1 ? 4 
     }
 }
 
-/* ---- forward, one band streaming its pairs back to back ----
- * For a query whose stripes fit one band (ns <= 8 waves): a persistent
- * workgroup takes the pairs at positions b, b+G, b+2G, ... of the launch
- * order (G = the grid) and runs them through its band without draining it:
- * wave w starts a pair's sweep when its own sweep of the previous pair ends,
- * 64 steps after wave w-1 does, so no wave idles between pairs and the band
- * fills and drains once per workgroup instead of once per pair.  A pair i
- * occupies wave w's steps u = T - 64w in [S_i, S_i + Ld_i + 64) (the first
- * only takes the row above), S_{i+1} = S_i + Ld_i + 64, the same for every
- * wave; when wave w needs the row above at a column of pair i, wave w-1 is
- * 64 steps further in the same pair, so the LDS hand-off is the per-pair
- * kernel's.  Every cell is computed as there; the pair's max F is the max of
- * the waves' maxima (non-negative, so an integer atomicMax on its bits). */
-template <int R>
-__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(R == 1 ? 4 : 1))) void k_map_fwd_pipe(ScoreCtx c, MapArgs m)
+/* ---- the streaming band kernels (k_map_*_pipe) ----
+ * For a query whose stripes fit one band (16 waves at one row per lane, 8
+ * beyond): a persistent workgroup takes the pairs at positions b, b+G, ... of
+ * the launch order (G = the grid) and runs them through its band without
+ * draining it: a pair i occupies wave w's stream steps [S_i, S_i + len_i), the
+ * same for every wave, len_i a multiple of four, and the waves are 68 steps
+ * apart in the order of the sweep.  Steps go in groups of four, unrolled: the
+ * four columns a wave's boundary row gains in a group are read by the next
+ * wave a group later, so one barrier per group suffices and the rows cross in
+ * small LDS rings addressed by the stream step.  A step waits for no memory:
+ * a profile's transitions pass through LDS in blocks of 64 columns fetched
+ * half a block ahead, S', F and B are loaded a group ahead, and a lane starts
+ * a pair from the column left of the matrix kept in its registers.
+ * Bound by VALU issue (forward about 250 operations a cell) with many pairs,
+ * by a pair's chain of steps with few. */
+constexpr int MLAG = 68;
+typedef const __attribute__((address_space(4))) int32_t* cip;
+
+/* a wave's window of a profile's transitions, column c at slot c & 127, 12
+ * words apart: 16-byte reads, the 8 lanes of one on distinct banks.  BWD:
+ * every class at c + 1, otherwise MI and II there */
+constexpr int MTW = 12;
+typedef float mf4 __attribute__((ext_vector_type(4)));
+template <bool BWD>
+struct MapWin {
+    float* w;
+    float v[7];
+    __device__ __forceinline__ void fetch(const float* T, size_t ntr, size_t db, int blk, int Ld, int lane)
+    {
+        const size_t b = db + (size_t)min(max(64 * blk + lane, 0), Ld - 1);
+#pragma unroll
+        for (int j = 0; j < 7; j++) v[j] = T[(size_t)j * ntr + b + (BWD || j == 1 || j == 4 ? 1 : 0)];
+    }
+    __device__ __forceinline__ void put(int blk, int lane)
+    {
+        mf4* p = (mf4*)(w + (((64 * blk) & 127) + lane) * MTW);
+        p[0] = mf4{v[0], v[1], v[2], v[3]}; p[1] = mf4{v[4], v[5], v[6], 0.0f};
+        wave_lds_sync();
+    }
+    __device__ __forceinline__ void get(int c, float* dt) const
+    {
+        const mf4* p = (const mf4*)(w + (c & 127) * MTW);
+        const mf4 a = p[0], b = p[1];
+        dt[0] = a[0]; dt[1] = a[1]; dt[2] = a[2]; dt[3] = a[3]; dt[4] = b[0]; dt[5] = b[1]; dt[6] = b[2];
+    }
+};
+
+/* a pair of the stream */
+struct MapPos { int pi, Ld; size_t db; int64_t foff, boff; };
+__device__ __forceinline__ MapPos map_pos(const ScoreCtx& c, const MapArgs& m, int o)
 {
-    __shared__ float hx[2][8][5];
+    MapPos p;
+    p.pi = __builtin_amdgcn_readfirstlane(((cip)m.order)[o]);
+    const MapPair mp = m.pairs[p.pi];
+    const int pro = __builtin_amdgcn_readfirstlane(mp.pro);
+    p.Ld = __builtin_amdgcn_readfirstlane(((cip)c.len)[pro]);
+    p.db = (size_t)(uint32_t)__builtin_amdgcn_readfirstlane(((cip)c.dist)[pro]) + (size_t)pro;
+    p.foff = mp.foff; p.boff = mp.boff;
+    return p;
+}
+
+/* forward cell: fcell with the sums of the row's MM transition and the row
+ * above's MM and MI given (um, ui; the diagonal's a step before: dgm, dgi).
+ * The largest term contributes e^0 = 1, so log's cut-off never applies */
+__device__ __forceinline__ S5 fcell_s(const S5& dg, float dgm, float dgi, const S5& up, float um, float ui, const S5& lf,
+                                      const float* qt, const float* dt, float sco, const float* tab)
+{
+    S5 n;
+    const float v1 = dgi + dt[3] + sco, v2 = dg.im + qt[3] + dt[0] + sco, v3 = dg.dn + qt[5] + dt[0] + sco,
+                v4 = dg.nd + qt[0] + dt[5] + sco, v5 = dgm + dt[0] + sco;
+    const float mx = fmaxf(fmaxf(fmaxf(v1, v2), fmaxf(v3, v4)), fmaxf(v5, 0.0f));
+    const float s = mexp(v1 - mx) + mexp(v2 - mx) + mexp(v3 - mx) + mexp(v4 - mx) + mexp(v5 - mx) + mexp(-mx);
+    n.mm = mlog(s) + mx;
+    n.mi = lse2(um + dt[1], ui + dt[4], tab);
+    n.im = lse2(lf.mm + qt[1] + dt[0], lf.im + qt[4] + dt[0], tab);
+    n.dn = lse2(up.mm + qt[2], up.dn + qt[6], tab);
+    n.nd = lse2(lf.mm + dt[2], lf.nd + dt[6], tab);
+    return n;
+}
+
+template <int R>
+__global__ __launch_bounds__(R == 1 ? 1024 : 512) void k_map_fwd_pipe(ScoreCtx c, MapArgs m)
+{
+    extern __shared__ __align__(16) float mwin[];
+    __shared__ __align__(16) float hx[R == 1 ? 16 : 8][16][5];
     __shared__ __align__(16) float tab[512];
     load_lse_tab(tab);
     int o0_, n_;
@@ -454,118 +523,150 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(R == 1 ? 4 
     const size_t ntr = (size_t)(c.npos + c.nprof);
     /* the band's length and the pairs' maxima cleared (each pair belongs to
      * this workgroup only) */
-    int TT = 64 * (NW - 1);
+    int TT = MLAG * (NW - 1);
     for (int j = (int)blockIdx.x; j < n_; j += G) {
         const int pj = m.order[o0_ + j];
-        TT += c.len[m.pairs[pj].pro] + 64;
+        TT += (c.len[m.pairs[pj].pro] + 66) & ~3;
         if (threadIdx.x == 0) {
             /* the max F, and the MAP DP's maximum key (k_map_dp_pipe) */
             m.stat[(size_t)pj * 4 + 0] = 0.0f;
             m.stat[(size_t)pj * 4 + 2] = 0.0f; m.stat[(size_t)pj * 4 + 3] = 0.0f;
         }
     }
+    TT = __builtin_amdgcn_readfirstlane(TT);
     __syncthreads();
-    int r[R]; bool valid[R]; float qt[R][7];
+    bool valid[R]; float qt[R][7];
+    S5 h0[R];                                     /* the column left of the matrix */
+    unsigned m31 = 0;                             /* rows whose diagonal at column 0 is row -1's */
 #pragma unroll
     for (int k = 0; k < R; k++) {
-        r[k] = s * 64 * R + R * lane + k;
-        valid[k] = r[k] < Lq;
+        const int r = s * 64 * R + R * lane + k, rr = min(r, Lq - 1);
+        valid[k] = r < Lq;
+        if ((r & 31) == 31) m31 |= 1u << k;
 #pragma unroll
-        for (int j = 0; j < 7; j++) qt[k][j] = valid[k] ? m.qtr[(size_t)j * c.Lpad + r[k]] : 0.0f;
+        for (int j = 0; j < 7; j++) qt[k][j] = valid[k] ? m.qtr[(size_t)j * c.Lpad + r] : 0.0f;
+        h0[k].mm = m.mleft[rr]; h0[k].mi = m.mleft[(size_t)Lq + rr]; h0[k].im = m.mleft[2 * (size_t)Lq + rr];
+        h0[k].dn = m.mleft[3 * (size_t)Lq + rr]; h0[k].nd = m.mleft[4 * (size_t)Lq + rr];
     }
-    /* the wave's current pair */
-    int jc = (int)blockIdx.x, S = 0, pi = 0, Ld = 0, nsteps = 0;
-    size_t db = 0;
-    const float* Sd = nullptr;
-    float* F = nullptr;
-    auto pair_at = [&](int j) {
-        pi = m.order[o0_ + j];
-        const MapPair mp = m.pairs[pi];
-        Ld = c.len[mp.pro]; nsteps = Ld + 63;
-        db = (size_t)c.dist[mp.pro] + mp.pro;
-        Sd = m.Sd + mp.foff; F = m.F + mp.foff;
-    };
-    pair_at(jc);
+    MapWin<false> tw;
+    tw.w = mwin + w * 128 * MTW;
+    int jc = (int)blockIdx.x, S = 0;
+    MapPos p = map_pos(c, m, o0_ + jc), q = p;
+    if (jc + G < n_) q = map_pos(c, m, o0_ + jc + G);
     float mymax = 0.0f;
-    S5 H[R];
-    S5 U = init5(), D = init5();
-    float sdn[R], dtn[7];
-    for (int T = 0; T < TT; T++) {
-        const int u = T - 64 * w;
-        if (u == S + nsteps + 1 && jc < n_) {
-            jc += G; S = u;
-            if (jc < n_) pair_at(jc);
-        }
-        const bool act = u >= S && jc < n_;
-        const int t = u - S - 1;                 /* -1 only takes the row above */
-        if (act && t == -1) {
+    S5 H[R], U = init5();
+    float um[R], ui[R], sn[R][4];
+    const float* Sd = m.Sd + p.foff;
+    auto load_s = [&](const float* sd, int t0, int nsteps) {
 #pragma unroll
-            for (int k = 0; k < R; k++) H[k] = init5();
-            U = init5(); D = init5();
-            mymax = 0.0f;
+        for (int u = 0; u < 4; u++)
 #pragma unroll
-            for (int k = 0; k < R; k++) sdn[k] = Sd[lsi<R>(s, 0, k, lane, nsteps)];
-            fwd_trn(m.trans, ntr, db, -lane, Ld, dtn);
-        }
-        if (act && t >= 0 && t < nsteps) {
-            const int cc = t - lane;
-            float sdc[R], dt[7];
-#pragma unroll
-            for (int k = 0; k < R; k++) sdc[k] = sdn[k];
-#pragma unroll
-            for (int j = 0; j < 7; j++) dt[j] = dtn[j];
-            if (t + 1 < nsteps) {
-#pragma unroll
-                for (int k = 0; k < R; k++) sdn[k] = Sd[lsi<R>(s, t + 1, k, lane, nsteps)];
-                fwd_trn(m.trans, ntr, db, cc + 1, Ld, dtn);
+            for (int k = 0; k < R; k++) sn[k][u] = sd[lsi<R>(s, min(t0 + u, nsteps - 1), k, lane, nsteps)];
+    };
+    load_s(Sd, 0, p.Ld + 63);
+    tw.fetch(m.trans, ntr, p.db, 0, p.Ld, lane);
+    for (int T0 = 0; T0 < TT; T0 += 4) {
+        const int u0 = T0 - MLAG * w;
+        if (u0 >= 0 && jc < n_) {
+            int t0 = u0 - S;
+            if (t0 == ((p.Ld + 66) & ~3)) {
+                jc += G; S = u0; t0 = 0;
+                p = q;
+                if (jc + G < n_) q = map_pos(c, m, o0_ + jc + G);
+                Sd = m.Sd + p.foff;
             }
-            if (cc >= 0 && cc < Ld) {
-                S5 prevk = D;
+            if (jc < n_) {
+                const int Ld = p.Ld, nsteps = Ld + 63;
+                float* F = m.F + p.foff;
+                float sc[R][4];
 #pragma unroll
-                for (int k = 0; k < R; k++) {
-                    S5 lf = H[k], dg = prevk;
-                    if (cc == 0) {
-                        const int rr = valid[k] ? r[k] : 0;
-                        lf.mm = m.mleft[0 * (size_t)Lq + rr]; lf.mi = m.mleft[1 * (size_t)Lq + rr];
-                        lf.im = m.mleft[2 * (size_t)Lq + rr]; lf.dn = m.mleft[3 * (size_t)Lq + rr];
-                        lf.nd = m.mleft[4 * (size_t)Lq + rr];
-                        dg.mm = m.mdiag[0 * (size_t)Lq + rr]; dg.mi = m.mdiag[1 * (size_t)Lq + rr];
-                        dg.im = m.mdiag[2 * (size_t)Lq + rr]; dg.dn = m.mdiag[3 * (size_t)Lq + rr];
-                        dg.nd = m.mdiag[4 * (size_t)Lq + rr];
+                for (int k = 0; k < R; k++)
+#pragma unroll
+                    for (int u = 0; u < 4; u++) sc[k][u] = sn[k][u];
+                if (t0 == 0) {
+                    tw.put(0, lane);
+                    U = init5();
+                    mymax = 0.0f;
+#pragma unroll
+                    for (int k = 0; k < R; k++) {
+                        H[k] = h0[k];
+                        um[k] = (k ? h0[k - 1].mm : U.mm) + qt[k][0];
+                        ui[k] = (k ? h0[k - 1].mi : U.mi) + qt[k][0];
                     }
-                    const S5 up = (k == 0) ? U : H[k - 1];
-                    prevk = H[k];
-                    const int64_t ix = lsi<R>(s, t, k, lane, nsteps);
-                    const S5 n = fcell(dg, up, lf, qt[k], dt, sdc[k], tab);
-                    H[k] = n;
-                    if (valid[k]) { F[ix] = n.mm; mymax = fmx(mymax, n.mm); }
                 }
-                if (lane == 63 && w + 1 < NW) {
-                    float* o = hx[T & 1][w];
-                    o[0] = H[R - 1].mm; o[1] = H[R - 1].mi; o[2] = H[R - 1].im;
-                    o[3] = H[R - 1].dn; o[4] = H[R - 1].nd;
+                if (t0 + 4 < nsteps) {
+                    load_s(Sd, t0 + 4, nsteps);
+                } else if (jc + G < n_) {
+                    load_s(m.Sd + q.foff, 0, q.Ld + 63);
+                    tw.fetch(m.trans, ntr, q.db, 0, q.Ld, lane);
                 }
-            }
-            if (t == nsteps - 1) {
-                /* the wave's sweep of the pair ends: its maximum */
-                float mx = mymax;
-                for (int off = 32; off >= 1; off >>= 1) mx = fmx(mx, __shfl_xor(mx, off));
-                if (lane == 0) atomicMax((unsigned int*)(m.stat + (size_t)pi * 4 + 0), __float_as_uint(mx));
+                if ((t0 & 63) == 32 && t0 + 32 < nsteps) tw.fetch(m.trans, ntr, p.db, (t0 >> 6) + 1, Ld, lane);
+                if ((t0 & 63) == 0 && t0 > 0) tw.put(t0 >> 6, lane);
+                /* the row above at columns t0 .. t0+3 */
+                float tp[20];
+                if (w == 0) {
+                    const S5 z = init5();
+#pragma unroll
+                    for (int i = 0; i < 20; i++) tp[i] = (i % 5) ? z.mi : z.mm;
+                } else {
+                    const mf4* o = (const mf4*)&hx[w - 1][u0 & 15][0];
+#pragma unroll
+                    for (int i = 0; i < 5; i++) {
+                        const mf4 x = o[i];
+#pragma unroll
+                        for (int j = 0; j < 4; j++) tp[4 * i + j] = x[j];
+                    }
+                }
+                auto step = [&](auto ALLC, auto UC) __attribute__((always_inline)) {
+                    constexpr bool ALL = decltype(ALLC)::value;
+                    constexpr int u = decltype(UC)::value;
+                    const int t = t0 + u, cc = t - lane;
+                    float dt[7];
+                    tw.get(cc, dt);
+                    S5 dg = U;
+                    U.mm = wave_shr1(H[R - 1].mm, tp[5 * u]); U.mi = wave_shr1(H[R - 1].mi, tp[5 * u + 1]);
+                    U.im = wave_shr1(H[R - 1].im, tp[5 * u + 2]); U.dn = wave_shr1(H[R - 1].dn, tp[5 * u + 3]);
+                    U.nd = wave_shr1(H[R - 1].nd, tp[5 * u + 4]);
+                    const bool in = ALL || (cc >= 0 && cc < Ld);
+                    S5 up = U;
+#pragma unroll
+                    for (int k = 0; k < R; k++) {
+                        const S5 old = H[k];
+                        float pm = um[k], pi = ui[k];
+                        um[k] = up.mm + qt[k][0]; ui[k] = up.mi + qt[k][0];
+                        if (in) {
+                            if (!ALL && cc == 0 && ((m31 >> k) & 1u)) { dg = init5(); pm = dg.mm + qt[k][0]; pi = dg.mi + qt[k][0]; }
+                            H[k] = fcell_s(dg, pm, pi, up, um[k], ui[k], old, qt[k], dt, sc[k][u], tab);
+                            if (valid[k]) mymax = fmx(mymax, H[k].mm);
+                        }
+                        /* words outside the matrix are written too and read by nobody */
+                        if (ALL || t < nsteps) F[lsi<R>(s, t, k, lane, nsteps)] = H[k].mm;
+                        dg = old; up = H[k];
+                    }
+                    if (lane == 63 && w + 1 < NW) {
+                        float* o = hx[w][(u0 + u + 1) & 15];
+                        const S5& e = H[R - 1];
+                        o[0] = e.mm; o[1] = e.mi; o[2] = e.im; o[3] = e.dn; o[4] = e.nd;
+                    }
+                };
+                using std::integral_constant;
+                if (t0 >= 64 && t0 + 3 < Ld) {
+                    step(std::true_type{}, integral_constant<int, 0>{}); step(std::true_type{}, integral_constant<int, 1>{});
+                    step(std::true_type{}, integral_constant<int, 2>{}); step(std::true_type{}, integral_constant<int, 3>{});
+                } else {
+                    step(std::false_type{}, integral_constant<int, 0>{}); step(std::false_type{}, integral_constant<int, 1>{});
+                    step(std::false_type{}, integral_constant<int, 2>{}); step(std::false_type{}, integral_constant<int, 3>{});
+                }
+                if (t0 + 4 >= nsteps) {
+                    /* the wave's sweep of the pair ends: its maximum (non-negative, so an
+                     * integer atomicMax on its bits) */
+                    float mx = mymax;
+                    for (int off = 32; off >= 1; off >>= 1) mx = fmx(mx, __shfl_xor(mx, off));
+                    if (lane == 0) atomicMax((unsigned int*)(m.stat + (size_t)p.pi * 4 + 0), __float_as_uint(mx));
+                }
             }
         }
         __syncthreads();
-        if (act && t >= -1 && t + 1 < nsteps) {
-            /* the row above the lane's first row at column t+1 - lane */
-            S5 tp = init5();
-            if (lane == 0 && w > 0 && t + 1 < Ld) {
-                const float* o = hx[T & 1][w - 1];
-                tp.mm = o[0]; tp.mi = o[1]; tp.im = o[2]; tp.dn = o[3]; tp.nd = o[4];
-            }
-            D = U;
-            U.mm = wave_shr1(H[R - 1].mm, tp.mm); U.mi = wave_shr1(H[R - 1].mi, tp.mi);
-            U.im = wave_shr1(H[R - 1].im, tp.im); U.dn = wave_shr1(H[R - 1].dn, tp.dn);
-            U.nd = wave_shr1(H[R - 1].nd, tp.nd);
-        }
     }
 }
 
@@ -584,13 +685,21 @@ __device__ int blk_ilim(int x0, int y, int Lq, int Ld) {
     return 32 <= xx ? 32 : xx;
 }
 
-/* 32 lanes per reference block: lane t holds column t of the block's rows,
- * the row sums use the same shfl_down tree as the reference, block sums are
- * added in the reference's block order */
+/* log Z, one workgroup per pair, 32 lanes per reference block: the reference
+ * adds a row's 32 terms by a tree over lanes (shfl_down 16, 8, 4, 2, 1), the
+ * rows one after another, the blocks in order.  Here lane i holds row i of the
+ * block whole and adds it up in registers by the same tree, so a row costs 31
+ * additions and no lane crossing (before: five dependent shuffles), and with
+ * one row per lane the block's cells at one step are one 128-byte read.  The
+ * rows' sums meet in LDS; the blocks' sums of up to MT_BLK blocks wait there
+ * for one thread to add them in order.  Bound by the exponentials.  200 pairs of
+ * 1,337 rows with up to 3,000 columns: 6.9 ms before */
+constexpr int MT_BLK = 2048;
 template <int R>
-__global__ __launch_bounds__(256) void k_map_total(ScoreCtx c, MapArgs m)
+__global__ __launch_bounds__(1024) void k_map_total(ScoreCtx c, MapArgs m)
 {
-    __shared__ float bsum[8];
+    __shared__ float bsum[MT_BLK];
+    __shared__ __align__(16) float rsum[32][32];
     int o0_, n_;
     map_range(m, &o0_, &n_);
     if ((int)blockIdx.x >= n_) return;            /* the grid covers the capacity */
@@ -604,66 +713,51 @@ __global__ __launch_bounds__(256) void k_map_total(ScoreCtx c, MapArgs m)
     int maxblk = (Lq + 31) / 32;
     { const int m2 = ((Ld + 64) + 63) / 64; if (m2 < maxblk) maxblk = m2; }
     const int nall = nblkdiags * maxblk;
-    const int g = threadIdx.x >> 5, t = threadIdx.x & 31;
+    const int g = threadIdx.x >> 5, i = threadIdx.x & 31, NG = (int)(blockDim.x >> 5);
     float total = 0.0f;
-    for (int base = 0; base < nall; base += 8) {
-        const int j = base + g;
-        float sum = 0.0f;
-        bool live = false;
-        int x0 = 0, y = 0;
-        if (j < nall) {
+    for (int cb = 0; cb < nall; cb += MT_BLK) {
+        const int ce = min(cb + MT_BLK, nall);
+        for (int j = cb + g; j < ce; j += NG) {
             const int dd = nblkdiags - 1 - j / maxblk, sb = j % maxblk;
+            int x0 = 0, y = 0;
             blk_origin(dd, sb, lastdiag, &x0, &y);
             const int ilim = blk_ilim(x0, y, Lq, Ld);
-            live = !(y < 0 || Lq <= y + 1 - 32 || Ld <= x0 || ilim < 1);
-        }
-        if (live) {
-            if constexpr (R == 1) {
-                /* one row per lane: the block's rows y-31..y are lanes ltop-31..ltop
-                 * of one stripe, and lane t's cells (y-i, x0+t+i) all sit at step
-                 * x0+t+ltop, 32 consecutive words: one 128-byte read per lane
-                 * instead of 32 scattered ones (same values, same sums) */
-                const int sI = y >> 6, ltop = y & 63, step = x0 + t + ltop;
+            float sum = 0.0f;
+            if (!(y < 0 || Lq <= y + 1 - 32 || Ld <= x0 || ilim < 1)) {
+                /* row y-i, columns x0+i .. x0+i+31 */
+                const int yy = y - i;
+                const bool row = 0 <= yy && yy < Lq;
+                const int yc = row ? yy : 0;
+                const int SL = 64 * R, sI = yc / SL, rr = yc - sI * SL, ln = rr / R, kk = rr - ln * R;
+                const float* Fr = F + lsi<R>(sI, 0, kk, ln, nsteps);
                 float v[32];
-                if (step >= 0 && step < nsteps) {
-                    const float4* src = (const float4*)(F + ((int64_t)sI * nsteps + step) * 64 + (ltop - 31));
 #pragma unroll
-                    for (int q = 0; q < 8; q++) {
-                        const float4 w4 = src[q];
-                        v[4 * q] = w4.x; v[4 * q + 1] = w4.y; v[4 * q + 2] = w4.z; v[4 * q + 3] = w4.w;
-                    }
-                } else {
+                for (int t = 0; t < 32; t++)
+                    v[t] = Fr[(int64_t)(min(max(x0 + i + t, 0), Ld - 1) + ln) * (64 * R)];
 #pragma unroll
-                    for (int q = 0; q < 32; q++) v[q] = 0.0f;
+                for (int t = 0; t < 32; t++) {
+                    const int xx = x0 + i + t;
+                    v[t] = (row && 0 <= xx && xx < Ld) ? mexp(v[t] - maxF) : 0.0f;
                 }
 #pragma unroll
-                for (int i = 0; i < 32; i++) {
-                    const int yy = y - i, xx = x0 + t + i;
-                    float nv = (0 <= yy && yy < Lq && 0 <= xx && xx < Ld) ? mexp(v[31 - i] - maxF) : 0.0f;
-                    for (int off = 16; off >= 1; off >>= 1) {
-                        const float o = __shfl_down(nv, off, 32);
-                        if (t + off < 32) nv += o;
-                    }
-                    sum += nv;
+                for (int off = 16; off >= 1; off >>= 1)
+#pragma unroll
+                    for (int t = 0; t < off; t++) v[t] += v[t + off];
+                rsum[g][i] = v[0];
+                wave_lds_sync();
+                const float4* rs = (const float4*)rsum[g];
+#pragma unroll
+                for (int q = 0; q < 8; q++) {
+                    const float4 x = rs[q];
+                    sum += x.x; sum += x.y; sum += x.z; sum += x.w;
                 }
-            } else {
-                for (int i = 0; i < 32; i++) {
-                    const int yy = y - i, xx = x0 + t + i;
-                    float nv = (0 <= yy && yy < Lq && 0 <= xx && xx < Ld) ? mexp(F[cell_lsi<R>(yy, xx, nsteps)] - maxF) : 0.0f;
-                    for (int off = 16; off >= 1; off >>= 1) {
-                        const float o = __shfl_down(nv, off, 32);
-                        if (t + off < 32) nv += o;
-                    }
-                    sum += nv;
-                }
+                wave_lds_sync();
             }
+            if (i == 0) bsum[j - cb] = sum;
         }
-        if (t == 0) bsum[g] = sum;
         __syncthreads();
-        if (threadIdx.x == 0) {
-            const int lim = (nall - base) < 8 ? (nall - base) : 8;
-            for (int k = 0; k < lim; k++) total += bsum[k];
-        }
+        if (threadIdx.x == 0)
+            for (int j = 0; j < ce - cb; j++) total += bsum[j];
         __syncthreads();
     }
     if (threadIdx.x == 0) m.stat[pi * 4 + 1] = mlog(total) + maxF;   /* logZ */
@@ -796,14 +890,14 @@ __global__ __launch_bounds__(512) void k_map_bwd(ScoreCtx c, MapArgs m)
 }
 
 /* ---- backward, one band streaming its pairs back to back ----
- * The reverse sweep of k_map_bwd with the pair stream of k_map_fwd_pipe:
- * wave w runs 64 steps behind wave w+1 (the stripe below), and a pair i
- * occupies wave w's steps u = T - 64(NW-1-w) in [S_i, S_i + Ld_i + 64), step
- * t = Ld_i + 63 - (u - S_i) (the first only takes the row below). */
+ * The reverse sweep of k_map_bwd: wave w runs behind wave w+1 (the stripe
+ * below); a pair's stream steps cover t = len-1 .. 0 with len >= Ld + 64, the
+ * steps past Ld + 62 only taking the row below. */
 template <int R>
-__global__ __launch_bounds__(512) void k_map_bwd_pipe(ScoreCtx c, MapArgs m)
+__global__ __launch_bounds__(R == 1 ? 1024 : 512) void k_map_bwd_pipe(ScoreCtx c, MapArgs m)
 {
-    __shared__ float hb[2][8][3];
+    extern __shared__ __align__(16) float mwin[];
+    __shared__ __align__(16) float hb[2][R == 1 ? 16 : 8][4][4];
     __shared__ __align__(16) float tab[512];
     load_lse_tab(tab);
     int o0_, n_;
@@ -812,106 +906,131 @@ __global__ __launch_bounds__(512) void k_map_bwd_pipe(ScoreCtx c, MapArgs m)
     if ((int)blockIdx.x >= n_) return;            /* uniform for the workgroup */
     const int lane = threadIdx.x & 63, NW = blockDim.x >> 6;
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
-    const int Lq = c.Lq, s = w, ns = NW;
+    const int Lq = c.Lq, s = w;
     const size_t ntr = (size_t)(c.npos + c.nprof);
-    int TT = 64 * (NW - 1);
-    for (int j = (int)blockIdx.x; j < n_; j += G) TT += c.len[m.pairs[m.order[o0_ + j]].pro] + 64;
-    int r[R]; bool valid[R]; float qt[R][7];
+    int TT = MLAG * (NW - 1);
+    for (int j = (int)blockIdx.x; j < n_; j += G) TT += (c.len[m.pairs[m.order[o0_ + j]].pro] + 67) & ~3;
+    TT = __builtin_amdgcn_readfirstlane(TT);
+    bool valid[R]; float qt[R][7];
 #pragma unroll
     for (int k = 0; k < R; k++) {
-        r[k] = s * 64 * R + R * lane + k;
-        valid[k] = r[k] < Lq;
+        const int r = s * 64 * R + R * lane + k;
+        valid[k] = r < Lq;
 #pragma unroll
-        for (int j = 0; j < 7; j++) qt[k][j] = valid[k] ? m.qtrb[(size_t)j * c.Lpad + r[k]] : 0.0f;
+        for (int j = 0; j < 7; j++) qt[k][j] = valid[k] ? m.qtrb[(size_t)j * c.Lpad + r] : 0.0f;
     }
-    const bool below = (s + 1 < ns);
-    int jc = (int)blockIdx.x, S = 0, Ld = 0, nsteps = 0;
-    size_t db = 0;
-    const float* Sd = nullptr;
-    float* Bm = nullptr;
-    auto pair_at = [&](int j) {
-        const MapPair mp = m.pairs[m.order[o0_ + j]];
-        Ld = c.len[mp.pro]; nsteps = Ld + 63;
-        db = (size_t)c.dist[mp.pro] + mp.pro;
-        Sd = m.Sd + mp.foff; Bm = m.B + mp.foff;
-    };
-    pair_at(jc);
+    const bool below = w + 1 < NW;
+    MapWin<true> tw;
+    tw.w = mwin + w * 128 * MTW;
+    int jc = (int)blockIdx.x, S = 0;
+    MapPos p = map_pos(c, m, o0_ + jc), q = p;
+    if (jc + G < n_) q = map_pos(c, m, o0_ + jc + G);
     S5 cur[R];
-    float scur[R];
-    float shmm = 0.0f, shmi = LP0, shdn = LP0, shs = LP0;
-    float spmm = 0.0f, sps = LP0;
-    float sdn[R], dxn[7];
-    for (int T = 0; T < TT; T++) {
-        const int u = T - 64 * (NW - 1 - w);
-        if (u == S + nsteps + 1 && jc < n_) {
-            jc += G; S = u;
-            if (jc < n_) pair_at(jc);
-        }
-        const bool act = u >= S && jc < n_;
-        const int t = nsteps - (u - S);          /* nsteps only takes the row below */
-        if (act && t == nsteps) {
+    float scur[R], sn[R][4];
+    float shmm = 0.0f, shmi = LP0, shdn = LP0, shs = LP0, spmm = 0.0f, sps = LP0;
+    const float* Sd = m.Sd + p.foff;
+    auto load_s = [&](const float* sd, int g0, int nsteps) {
 #pragma unroll
-            for (int k = 0; k < R; k++) { cur[k] = init5(); scur[k] = LP0; }
-            shmm = 0.0f; shmi = LP0; shdn = LP0; shs = LP0;
-            spmm = 0.0f; sps = LP0;
+        for (int u = 0; u < 4; u++)
 #pragma unroll
-            for (int k = 0; k < R; k++) sdn[k] = Sd[lsi<R>(s, nsteps - 1, k, lane, nsteps)];
-            bwd_trn(m.trans, ntr, db, nsteps - 1 - lane, Ld, dxn);
-        }
-        if (act && t >= 0 && t < nsteps) {
-            const int cc = t - lane;
-            float sdc[R], dx[7];
-#pragma unroll
-            for (int k = 0; k < R; k++) sdc[k] = sdn[k];
-#pragma unroll
-            for (int j = 0; j < 7; j++) dx[j] = dxn[j];
-            if (t > 0) {
-#pragma unroll
-                for (int k = 0; k < R; k++) sdn[k] = Sd[lsi<R>(s, t - 1, k, lane, nsteps)];
-                bwd_trn(m.trans, ntr, db, cc - 1, Ld, dxn);
+            for (int k = 0; k < R; k++) sn[k][u] = sd[lsi<R>(s, min(g0 + u, nsteps - 1), k, lane, nsteps)];
+    };
+    load_s(Sd, ((p.Ld + 67) & ~3) - 4, p.Ld + 63);
+    tw.fetch(m.trans, ntr, p.db, (p.Ld - 1) >> 6, p.Ld, lane);
+    for (int T0 = 0; T0 < TT; T0 += 4) {
+        const int u0 = T0 - MLAG * (NW - 1 - w), par = (T0 >> 2) & 1;
+        if (u0 >= 0 && jc < n_) {
+            int len = (p.Ld + 67) & ~3;
+            if (u0 - S == len) {
+                jc += G; S = u0;
+                p = q;
+                if (jc + G < n_) q = map_pos(c, m, o0_ + jc + G);
+                Sd = m.Sd + p.foff;
+                len = (p.Ld + 67) & ~3;
             }
-            if (cc >= 0 && cc < Ld) {
-                float nmi = shmi, ndn = shdn;
-                float omm = spmm, os = sps;
+            if (jc < n_) {
+                const int Ld = p.Ld, nsteps = Ld + 63, bl = (Ld - 1) >> 6;
+                const int g0 = len - 4 - (u0 - S);
+                float* Bm = m.B + p.foff;
+                float sc[R][4];
 #pragma unroll
-                for (int k = R - 1; k >= 0; k--) {
-                    const float dgmm = omm, dsc = os;
-                    const S5 rt = cur[k];
-                    omm = cur[k].mm; os = scur[k];
-                    const int64_t ix = lsi<R>(s, t, k, lane, nsteps);
-                    const float sk = sdc[k];
-                    S5 n = init5();
-                    if (valid[k]) {
-                        n = bcell(dgmm, nmi, ndn, rt, qt[k], dx, dsc, tab);
-                        Bm[ix] = n.mm;
+                for (int k = 0; k < R; k++)
+#pragma unroll
+                    for (int u = 0; u < 4; u++) sc[k][u] = sn[k][u];
+                if (u0 == S) {
+                    tw.put(bl, lane);
+                    tw.fetch(m.trans, ntr, p.db, bl - 1, Ld, lane);
+#pragma unroll
+                    for (int k = 0; k < R; k++) { cur[k] = init5(); scur[k] = LP0; }
+                    shmm = 0.0f; shmi = LP0; shdn = LP0; shs = LP0; spmm = 0.0f; sps = LP0;
+                }
+                if ((g0 & 63) == 60 && (g0 >> 6) <= bl) tw.put((g0 >> 6) - 1, lane);
+                if ((g0 & 63) == 28 && (g0 >> 6) - 2 < bl - 1) tw.fetch(m.trans, ntr, p.db, (g0 >> 6) - 2, Ld, lane);
+                if (g0 > 0) {
+                    load_s(Sd, g0 - 4, nsteps);
+                } else if (jc + G < n_) {
+                    load_s(m.Sd + q.foff, ((q.Ld + 67) & ~3) - 4, q.Ld + 63);
+                    tw.fetch(m.trans, ntr, q.db, (q.Ld - 1) >> 6, q.Ld, lane);
+                }
+                auto step = [&](auto ALLC, auto UC) __attribute__((always_inline)) {
+                    constexpr bool ALL = decltype(ALLC)::value;
+                    constexpr int u = decltype(UC)::value;
+                    const int t = g0 + u, cc = t - lane;
+                    if (ALL || t < nsteps) {
+                        float dx[7];
+                        tw.get(cc, dx);
+                        if (ALL || (cc >= 0 && cc < Ld)) {
+                            float nmi = shmi, ndn = shdn;     /* new B of row k+1 at column c */
+                            float omm = spmm, os = sps;       /* old B_MM, S' of row k+1 at column c+1 */
+#pragma unroll
+                            for (int k = R - 1; k >= 0; k--) {
+                                const float dgmm = omm, dsc = os;
+                                const S5 rt = cur[k];
+                                omm = cur[k].mm; os = scur[k];
+                                S5 n = init5();
+                                if (valid[k]) {
+                                    n = bcell(dgmm, nmi, ndn, rt, qt[k], dx, dsc, tab);
+                                    Bm[lsi<R>(s, t, k, lane, nsteps)] = n.mm;
+                                }
+                                cur[k] = n; scur[k] = sc[k][u];
+                                nmi = n.mi; ndn = n.dn;
+                            }
+                        } else {
+#pragma unroll
+                            for (int k = 0; k < R; k++) { cur[k] = init5(); scur[k] = LP0; }
+                        }
+                        if (lane == 0 && w > 0) {
+                            float* o = hb[par][w][u];
+                            o[0] = cur[0].mm; o[1] = cur[0].mi; o[2] = cur[0].dn; o[3] = scur[0];
+                        }
                     }
-                    cur[k] = n; scur[k] = sk;
-                    nmi = n.mi; ndn = n.dn;
+                    if (ALL || (t >= 1 && t <= nsteps)) {
+                        /* the row below for step t-1: lane l+1's first row, or for lane 63
+                         * the stripe below at column t-1-63 */
+                        float obmm = 0.0f, obmi = LP0, obdn = LP0, obs = LP0;
+                        const int cb = t - 1 - 63;
+                        if (below && cb >= 0 && cb < Ld) {
+                            const mf4 o = *(const mf4*)hb[par ^ 1][w + 1][u];
+                            obmm = o[0]; obmi = o[1]; obdn = o[2]; obs = o[3];
+                        }
+                        spmm = shmm; sps = shs;
+                        shmm = wave_shl1(cur[0].mm, obmm);
+                        shmi = wave_shl1(cur[0].mi, obmi);
+                        shdn = wave_shl1(cur[0].dn, obdn);
+                        shs = wave_shl1(scur[0], obs);
+                    }
+                };
+                using std::integral_constant;
+                if (g0 >= 64 && g0 + 3 < Ld) {
+                    step(std::true_type{}, integral_constant<int, 3>{}); step(std::true_type{}, integral_constant<int, 2>{});
+                    step(std::true_type{}, integral_constant<int, 1>{}); step(std::true_type{}, integral_constant<int, 0>{});
+                } else {
+                    step(std::false_type{}, integral_constant<int, 3>{}); step(std::false_type{}, integral_constant<int, 2>{});
+                    step(std::false_type{}, integral_constant<int, 1>{}); step(std::false_type{}, integral_constant<int, 0>{});
                 }
-                if (lane == 0 && w > 0) {
-                    float* o = hb[T & 1][w];
-                    o[0] = cur[0].mm; o[1] = cur[0].mi; o[2] = cur[0].dn;
-                }
-            } else {
-#pragma unroll
-                for (int k = 0; k < R; k++) { cur[k] = init5(); scur[k] = LP0; }
             }
         }
         __syncthreads();
-        if (act && t >= 1 && t <= nsteps) {
-            float obmm = 0.0f, obmi = LP0, obdn = LP0, obs = LP0;
-            const int cb = t - 1 - 63;
-            if (lane == 63 && below && cb >= 0 && cb < Ld) {
-                const float* o = hb[T & 1][w + 1];
-                obmm = o[0]; obmi = o[1]; obdn = o[2];
-                obs = Sd[lsi<R>(s + 1, cb, 0, 0, nsteps)];
-            }
-            spmm = shmm; sps = shs;
-            shmm = wave_shl1(cur[0].mm, obmm);
-            shmi = wave_shl1(cur[0].mi, obmi);
-            shdn = wave_shl1(cur[0].dn, obdn);
-            shs = wave_shl1(scur[0], obs);
-        }
     }
 }
 
@@ -1061,9 +1180,9 @@ __device__ __forceinline__ unsigned long long dp_key(float v, int x, int y)
 }
 
 template <int R>
-__global__ __launch_bounds__(512) void k_map_dp_pipe(ScoreCtx c, MapArgs m)
+__global__ __launch_bounds__(R == 1 ? 1024 : 512) void k_map_dp_pipe(ScoreCtx c, MapArgs m)
 {
-    __shared__ float hv[2][8];
+    __shared__ __align__(16) float hv[R == 1 ? 16 : 8][16];
     int o0_, n_;
     map_range(m, &o0_, &n_);
     const int G = (int)gridDim.x;
@@ -1072,114 +1191,113 @@ __global__ __launch_bounds__(512) void k_map_dp_pipe(ScoreCtx c, MapArgs m)
     const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int Lq = c.Lq, s = w;
     const float minpp = m.minpp, gapreg = m.minpp * 0.5f;
-    int TT = 64 * (NW - 1);
-    for (int j = (int)blockIdx.x; j < n_; j += G) TT += c.len[m.pairs[m.order[o0_ + j]].pro] + 64;
+    int TT = MLAG * (NW - 1);
+    for (int j = (int)blockIdx.x; j < n_; j += G) TT += (c.len[m.pairs[m.order[o0_ + j]].pro] + 66) & ~3;
+    TT = __builtin_amdgcn_readfirstlane(TT);
     int r[R];
 #pragma unroll
     for (int k = 0; k < R; k++) r[k] = s * 64 * R + R * lane + k;
-    int jc = (int)blockIdx.x, S = 0, pi = 0, Ld = 0, nsteps = 0, e = 0, tl = 0;
+    int jc = (int)blockIdx.x, S = 0, e = 0, tl = 0;
+    MapPos p = map_pos(c, m, o0_ + jc), q = p;
+    if (jc + G < n_) q = map_pos(c, m, o0_ + jc + G);
     float logZ = 0.0f;
-    const float* Fm = nullptr;
-    const float* Bm = nullptr;
-    char* bt = nullptr;
-    auto pair_at = [&](int j) {
-        pi = m.order[o0_ + j];
-        const MapPair mp = m.pairs[pi];
-        Ld = c.len[mp.pro]; nsteps = Ld + 63;
-        Fm = m.F + mp.foff; Bm = m.B + mp.foff; bt = m.btck + mp.boff;
-        logZ = m.stat[(size_t)pi * 4 + 1];
-        e = (int)rintf(0.34f * (float)(Lq > Ld ? Lq : Ld));
-        if (e > 60) e = 60;
-        tl = (Ld - 1) % 32;
-    };
-    pair_at(jc);
     float best = 0.0f; int bx = 0, by = 0;
-    float V[R], fn_[R], bn_[R];
-    float U = 0.0f, D = 0.0f;
-    for (int T = 0; T < TT; T++) {
-        const int u = T - 64 * w;
-        if (u == S + nsteps + 1 && jc < n_) {
-            jc += G; S = u;
-            if (jc < n_) pair_at(jc);
-        }
-        const bool act = u >= S && jc < n_;
-        const int t = u - S - 1;
-        if (act && t == -1) {
+    float V[R], U = 0.0f, fn_[R][4], bn_[R][4];
+    auto load_fb = [&](const MapPos& x, int t0) {
+        const int ns_ = x.Ld + 63;
 #pragma unroll
-            for (int k = 0; k < R; k++) V[k] = 0.0f;
-            U = 0.0f; D = 0.0f;
-            best = 0.0f; bx = 0; by = 0;
+        for (int u = 0; u < 4; u++)
 #pragma unroll
             for (int k = 0; k < R; k++) {
-                const int64_t ix = lsi<R>(s, 0, k, lane, nsteps);
-                fn_[k] = Fm[ix]; bn_[k] = Bm[ix];
+                const int64_t ix = x.foff + lsi<R>(s, min(t0 + u, ns_ - 1), k, lane, ns_);
+                fn_[k][u] = m.F[ix]; bn_[k][u] = m.B[ix];
             }
-        }
-        if (act && t >= 0 && t < nsteps) {
-            const int cc = t - lane;
-            float fbc[R];
-#pragma unroll
-            for (int k = 0; k < R; k++) fbc[k] = fn_[k] + bn_[k];
-            if (t + 1 < nsteps) {
-#pragma unroll
-                for (int k = 0; k < R; k++) {
-                    const int64_t ix = lsi<R>(s, t + 1, k, lane, nsteps);
-                    fn_[k] = Fm[ix]; bn_[k] = Bm[ix];
-                }
+    };
+    load_fb(p, 0);
+    for (int T0 = 0; T0 < TT; T0 += 4) {
+        const int u0 = T0 - MLAG * w;
+        if (u0 >= 0 && jc < n_) {
+            int t0 = u0 - S;
+            if (t0 == ((p.Ld + 66) & ~3)) {
+                jc += G; S = u0; t0 = 0;
+                p = q;
+                if (jc + G < n_) q = map_pos(c, m, o0_ + jc + G);
             }
-            if (cc >= 0 && cc < Ld) {
-                float prevk = D;
+            if (jc < n_) {
+                const int Ld = p.Ld, nsteps = Ld + 63;
+                char* bt = m.btck + p.boff;
+                if (t0 == 0) {
 #pragma unroll
-                for (int k = 0; k < R; k++) {
-                    const int y = r[k];
-                    const int64_t ix = lsi<R>(s, t, k, lane, nsteps);
-                    const bool ok = in_valid(Lq, Ld, e, y, cc);
-                    const float fb = ok ? fbc[k] : 0.0f;
-                    const float dgv = (y > 0 && cc > 0) ? prevk : 0.0f;
-                    const bool upzero = (cc == Ld - 1 && tl != 31 && (y % 32) == 31 - tl);
-                    const float upv = (y > 0 && !upzero) ? ((k == 0) ? U : V[k - 1]) : 0.0f;
-                    const float lfv = (cc > 0) ? V[k] : 0.0f;
-                    prevk = V[k];
-                    char bc = 0;
-                    float v = dgv + mexp(fb - logZ) - minpp;
-                    if (v > 0.0f) bc = 3; else v = 0.0f;
-                    if (ok && v > 0.0f && better(v, cc, y, best, bx, by)) { best = v; bx = cc; by = y; }
-                    const float uu = upv - gapreg; if (v < uu) { v = uu; bc = 2; }
-                    const float l = lfv - gapreg; if (v < l) { v = l; bc = 1; }
-                    V[k] = v;
-                    if (y < Lq) bt[ix] = bc;
+                    for (int k = 0; k < R; k++) V[k] = 0.0f;
+                    U = 0.0f;
+                    best = 0.0f; bx = 0; by = 0;
+                    logZ = m.stat[(size_t)p.pi * 4 + 1];
+                    e = (int)rintf(0.34f * (float)(Lq > Ld ? Lq : Ld));
+                    if (e > 60) e = 60;
+                    tl = (Ld - 1) % 32;
                 }
-                if (lane == 63 && w + 1 < NW) hv[T & 1][w] = V[R - 1];
-            }
-            if (t == nsteps - 1) {
-                /* the wave's sweep of the pair ends: its canonical maximum */
-                unsigned long long key = dp_key(best, bx, by);
-                for (int off = 32; off >= 1; off >>= 1) {
-                    const unsigned long long o = __shfl_xor(key, off);
-                    key = o > key ? o : key;
+                float fb_[R][4];
+#pragma unroll
+                for (int k = 0; k < R; k++)
+#pragma unroll
+                    for (int u = 0; u < 4; u++) fb_[k][u] = fn_[k][u] + bn_[k][u];
+                if (t0 + 4 < nsteps) load_fb(p, t0 + 4);
+                else if (jc + G < n_) load_fb(q, 0);
+                mf4 tp = mf4{0.0f, 0.0f, 0.0f, 0.0f};        /* the row above at columns t0 .. t0+3 */
+                if (w > 0) tp = *(const mf4*)&hv[w - 1][u0 & 15];
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const int t = t0 + u, cc = t - lane;
+                    const float D = U;
+                    U = wave_shr1(V[R - 1], tp[u]);
+                    if (cc >= 0 && cc < Ld) {
+                        float prevk = D;
+#pragma unroll
+                        for (int k = 0; k < R; k++) {
+                            const int y = r[k];
+                            const bool ok = in_valid(Lq, Ld, e, y, cc);
+                            const float fb = ok ? fb_[k][u] : 0.0f;
+                            const float dgv = (y > 0 && cc > 0) ? prevk : 0.0f;
+                            const bool upzero = (cc == Ld - 1 && tl != 31 && (y % 32) == 31 - tl);
+                            const float upv = (y > 0 && !upzero) ? ((k == 0) ? U : V[k - 1]) : 0.0f;
+                            const float lfv = (cc > 0) ? V[k] : 0.0f;
+                            prevk = V[k];
+                            char bc = 0;
+                            float v = dgv + mexp(fb - logZ) - minpp;
+                            if (v > 0.0f) bc = 3; else v = 0.0f;
+                            if (ok && v > 0.0f && better(v, cc, y, best, bx, by)) { best = v; bx = cc; by = y; }
+                            const float uu = upv - gapreg; if (v < uu) { v = uu; bc = 2; }
+                            const float l = lfv - gapreg; if (v < l) { v = l; bc = 1; }
+                            V[k] = v;
+                            if (y < Lq) bt[lsi<R>(s, t, k, lane, nsteps)] = bc;
+                        }
+                    }
+                    if (lane == 63 && w + 1 < NW) hv[w][(u0 + u + 1) & 15] = V[R - 1];
                 }
-                if (lane == 0) {
-                    unsigned long long* kp = (unsigned long long*)(m.stat + (size_t)pi * 4 + 2);
-                    const unsigned long long old = atomicMax(kp, key);
-                    if (w == NW - 1) {
-                        const unsigned long long k2 = old > key ? old : key;
-                        const float bv = k2 ? __uint_as_float((uint32_t)(k2 >> 32)) : 0.0f;
-                        const uint32_t xy = k2 ? 0xFFFFFFFFu - (uint32_t)k2 : 0u;
-                        int32_t* o = m.res + (size_t)pi * 8;
-                        o[5] = (int32_t)(bv > 0.0f ? xy : 0u);
-                        o[6] = __float_as_int(bv);
-                        o[7] = __float_as_int(logZ);
+                if (t0 + 4 >= nsteps) {
+                    /* the wave's sweep of the pair ends: its canonical maximum */
+                    unsigned long long key = dp_key(best, bx, by);
+                    for (int off = 32; off >= 1; off >>= 1) {
+                        const unsigned long long o = __shfl_xor(key, off);
+                        key = o > key ? o : key;
+                    }
+                    if (lane == 0) {
+                        unsigned long long* kp = (unsigned long long*)(m.stat + (size_t)p.pi * 4 + 2);
+                        const unsigned long long old = atomicMax(kp, key);
+                        if (w == NW - 1) {
+                            const unsigned long long k2 = old > key ? old : key;
+                            const float bv = k2 ? __uint_as_float((uint32_t)(k2 >> 32)) : 0.0f;
+                            const uint32_t xy = k2 ? 0xFFFFFFFFu - (uint32_t)k2 : 0u;
+                            int32_t* o = m.res + (size_t)p.pi * 8;
+                            o[5] = (int32_t)(bv > 0.0f ? xy : 0u);
+                            o[6] = __float_as_int(bv);
+                            o[7] = __float_as_int(logZ);
+                        }
                     }
                 }
             }
         }
         __syncthreads();
-        if (act && t >= -1 && t + 1 < nsteps) {
-            float tp = 0.0f;
-            if (lane == 0 && w > 0 && t + 1 < Ld) tp = hv[T & 1][w - 1];
-            D = U;
-            U = wave_shr1(V[R - 1], tp);
-        }
     }
 }
 
@@ -1210,12 +1328,12 @@ __global__ __launch_bounds__(64) void k_map_final(ScoreCtx c, MapArgs m, int npa
 /* persistent grid of the streaming band kernels: the workgroups that fit
  * the device at once (at most npairs) */
 template <class K>
-int pipe_grid(K kern, int nw, int npairs)
+int pipe_grid(K kern, int nw, int npairs, size_t lds)
 {
     int dev = 0, ncu = 0, per = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
         hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1 ||
-        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, 64 * nw, 0) != hipSuccess || per < 1)
+        hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kern, 64 * nw, lds) != hipSuccess || per < 1)
         return npairs;
     const int g = per * ncu;
     return g < npairs ? g : npairs;
@@ -1239,14 +1357,17 @@ hipError_t launch_r(const ScoreCtx& c, const MapArgs& m0, int npairs, hipStream_
         if (c.cvs.wgt > 0.0f) hipLaunchKernelGGL((k_map_score<R, true>), dim3(grid_s), dim3(256), 0, stream, c, m);
         else hipLaunchKernelGGL((k_map_score<R, false>), dim3(grid_s), dim3(256), 0, stream, c, m);
     }
-    /* one band per query (its stripes fit 8 waves): the forward and backward
-     * passes stream each workgroup's pairs through its band */
+    /* one band per query: the passes stream each workgroup's pairs through it */
     const bool pipe = m.pipe && m.nw == m.ns;
-    const int gf = pipe ? pipe_grid(k_map_fwd_pipe<R>, m.nw, npairs) : npairs;
-    const int gb = pipe ? pipe_grid(k_map_bwd_pipe<R>, m.nw, npairs) : npairs;
+    const size_t lds = sizeof(float) * (size_t)m.nw * 128 * MTW;      /* the waves' transition windows */
+    C2_LDS_LIMIT_ONCE(k_map_fwd_pipe<R>, 16 * 128 * MTW * sizeof(float));
+    C2_LDS_LIMIT_ONCE(k_map_bwd_pipe<R>, 16 * 128 * MTW * sizeof(float));
+    const int gf = pipe ? pipe_grid(k_map_fwd_pipe<R>, m.nw, npairs, lds) : npairs;
+    const int gb = pipe ? pipe_grid(k_map_bwd_pipe<R>, m.nw, npairs, lds) : npairs;
+    const int wgb = wg > 512 ? 512 : wg;                              /* bands of the per-pair kernels */
     auto bwd = [&](hipStream_t st) {
-        if (pipe) hipLaunchKernelGGL((k_map_bwd_pipe<R>), dim3(gb), dim3(wg), 0, st, c, m);
-        else hipLaunchKernelGGL((k_map_bwd<R>), dim3(npairs), dim3(wg), 0, st, c, m);
+        if (pipe) hipLaunchKernelGGL((k_map_bwd_pipe<R>), dim3(gb), dim3(wg), lds, st, c, m);
+        else hipLaunchKernelGGL((k_map_bwd<R>), dim3(npairs), dim3(wgb), 0, st, c, m);
     };
     if (bstream) {
         if ((e = hipEventRecord(fork, stream)) != hipSuccess) return e;
@@ -1254,17 +1375,17 @@ hipError_t launch_r(const ScoreCtx& c, const MapArgs& m0, int npairs, hipStream_
         bwd(bstream);
         if ((e = hipEventRecord(join, bstream)) != hipSuccess) return e;
     }
-    if (pipe) hipLaunchKernelGGL((k_map_fwd_pipe<R>), dim3(gf), dim3(wg), 0, stream, c, m);
-    else hipLaunchKernelGGL((k_map_fwd<R>), dim3(npairs), dim3(wg), 0, stream, c, m);
-    hipLaunchKernelGGL((k_map_total<R>), dim3(npairs), dim3(256), 0, stream, c, m);
+    if (pipe) hipLaunchKernelGGL((k_map_fwd_pipe<R>), dim3(gf), dim3(wg), lds, stream, c, m);
+    else hipLaunchKernelGGL((k_map_fwd<R>), dim3(npairs), dim3(wgb), 0, stream, c, m);
+    hipLaunchKernelGGL((k_map_total<R>), dim3(npairs), dim3(npairs > 1024 ? 256 : 1024), 0, stream, c, m);
     if (bstream) {
         if ((e = hipStreamWaitEvent(stream, join, 0)) != hipSuccess) return e;
     } else {
         bwd(stream);
     }
-    if (pipe) hipLaunchKernelGGL((k_map_dp_pipe<R>), dim3(pipe_grid(k_map_dp_pipe<R>, m.nw, npairs)), dim3(wg), 0,
+    if (pipe) hipLaunchKernelGGL((k_map_dp_pipe<R>), dim3(pipe_grid(k_map_dp_pipe<R>, m.nw, npairs, 0)), dim3(wg), 0,
                                  stream, c, m);
-    else hipLaunchKernelGGL((k_map_dp<R>), dim3(npairs), dim3(wg), 0, stream, c, m);
+    else hipLaunchKernelGGL((k_map_dp<R>), dim3(npairs), dim3(wgb), 0, stream, c, m);
     hipLaunchKernelGGL((k_map_final<R>), dim3(npairs), dim3(64), 0, stream, c, m, npairs);
     return hipGetLastError();
 }
@@ -1274,15 +1395,16 @@ hipError_t launch_r(const ScoreCtx& c, const MapArgs& m0, int npairs, hipStream_
 int64_t c2_map_cells(int R, int nstripes, int Ld) { return (int64_t)nstripes * (Ld + 63) * R * 64; }
 int64_t c2_map_hand(int nstripes, int Ld) { return (int64_t)nstripes * 5 * Ld + 4 * (int64_t)Ld; }
 
-/* rows per lane so that one band of at most 8 waves covers the query when
- * it can (R <= 5); waves = stripes of the first band */
+/* one row per lane while a workgroup's 16 waves cover the query (a pair's
+ * chain of steps is then the shortest), beyond 1,024 rows as many rows per
+ * lane as let 8 waves cover it (R <= 5); waves = stripes of the first band */
 void c2_map_geometry(int Lq, int* R, int* ns, int* nw)
 {
-    int r = (Lq + 511) / 512;
-    if (r < 1) r = 1;
+    int r = Lq <= 1024 ? 1 : (Lq + 511) / 512;
     if (r > 5) r = 5;
-    const int n = (Lq + 64 * r - 1) / (64 * r);
-    *R = r; *ns = n; *nw = n < 8 ? n : 8;
+    int n = (Lq + 64 * r - 1) / (64 * r);
+    if (n < 1) n = 1;
+    *R = r; *ns = n; *nw = r == 1 ? n : (n < 8 ? n : 8);
 }
 
 void c2_map_geometry_short(int Lq, int rmax, int* R, int* ns, int* nw)
@@ -1300,7 +1422,7 @@ hipError_t c2_launch_map(const ScoreCtx& c, const MapArgs& m, int npairs, hipStr
                          hipStream_t bstream, hipEvent_t fork, hipEvent_t join)
 {
     if (npairs <= 0) return hipSuccess;
-    if (m.nw < 1 || m.nw > 8 || m.ns < 1 || !m.order || !m.sitems || !m.B ||
+    if (m.nw < 1 || m.nw > (m.R == 1 ? 16 : 8) || m.ns < 1 || !m.order || !m.sitems || !m.B ||
         (!m.dcnt && m.nsitems < npairs * m.ns))
         return hipErrorInvalidValue;
     if (bstream && (!fork || !join)) return hipErrorInvalidValue;

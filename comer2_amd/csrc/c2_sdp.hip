@@ -19,11 +19,11 @@
  * hardware exp2/log2.
  *
  * Decomposition: a pair is cut into stripes of 64 query rows, one wave per
- * stripe, lane l owning row l and processing column t-l at step t, the row above arriving from lane l-1 by DPP wave_shr:1 (forward) and
- * the row below from lane l+1 by wave_shl:1 (adjoint).  A workgroup takes a
- * band of up to 4 stripes that advance in lockstep, passing their boundary
- * row through LDS.  Bands of one
- * pair run in different workgroups at once: the boundary row goes through
+ * stripe, lane l owning row l and processing column t-l at step t, the row
+ * above arriving from lane l-1 by DPP wave_shr:1 (forward) and the row below
+ * from lane l+1 by wave_shl:1 (adjoint).  A workgroup takes a band of up to 4
+ * stripes that advance in lockstep, passing their boundary row through LDS.
+ * Bands of one pair run in different workgroups at once: the boundary row goes through
  * memory as words that a launch first sets to a value no state has, so a
  * word is its own arrival flag and the band after polls 64 columns at a time
  * (agent-scope relaxed atomics, no fences).  Workgroups take (pair, band)
@@ -41,10 +41,10 @@
  * columns at a time, and the terms that leave the matrix's edges are added
  * after the sweep.  One row per lane: the padding of a pair's last stripe is
  * at most 63 rows, and a step's chain is one cell.  Every cell's operations
- * and their order are those of the one-workgroup-per-pair sweep.  Measured (before: stripes
- * of 320 rows, one workgroup per pair, inputs loaded in the step that used
- * them): 1,024 pairs of 50-600, forward + adjoint 8.04 -> 4.03 ms; 24 pairs
- * of 2,000-5,000 with checkpoints 135 -> 21.5 ms.
+ * and their order are those of the one-workgroup-per-pair sweep.  Measured
+ * (before: stripes of 320 rows, one workgroup per pair, inputs loaded in the
+ * step that used them): 1,024 pairs of 50-600, forward + adjoint 8.01 -> 3.86
+ * ms; 24 pairs of 2,000-5,000 with checkpoints 143.7 -> 22.2 ms.
  */
 #include <algorithm>
 #include <type_traits>
