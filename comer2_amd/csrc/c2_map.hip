@@ -8,7 +8,8 @@
  * (CuBatchMAPDP_map_final.cu:63-431).
  *
  * Decomposition: one workgroup per realigned pair (longest first), one
- * wave per stripe of 64*R query rows, up to 8 stripes in flight; inside a
+ * wave per stripe of 64*R query rows, up to 8 stripes in flight (16 at one
+ * row per lane in the streaming kernels below); inside a
  * wave the lane-rows wavefront of the phase-1 kernel: lane l owns rows
  * R*l..R*l+R-1 and handles column t-l at step t; the row above (forward and
  * MAP DP) arrives from lane l-1 by DPP wave_shr:1, the row below (backward)
@@ -439,8 +440,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(R == 1 ? 4 
  * a profile's transitions pass through LDS in blocks of 64 columns fetched
  * half a block ahead, S', F and B are loaded a group ahead, and a lane starts
  * a pair from the column left of the matrix kept in its registers.
- * Bound by VALU issue (forward about 250 operations a cell) with many pairs,
- * by a pair's chain of steps with few. */
+ * Bound by VALU issue with many pairs, by a pair's chain of steps with few.
+ * The longer of a call's two forward launches, against a step at a time with
+ * loads and a barrier in each: 100 pairs x 150 rows 1.23 -> 0.91 ms, 2,000 x
+ * 300 rows 3.19 -> 2.33 ms, 200 x 1,337 rows (R = 3) 8.7 -> 6.6 ms. */
 constexpr int MLAG = 68;
 typedef const __attribute__((address_space(4))) int32_t* cip;
 
@@ -693,7 +696,7 @@ __device__ int blk_ilim(int x0, int y, int Lq, int Ld) {
  * one row per lane the block's cells at one step are one 128-byte read.  The
  * rows' sums meet in LDS; the blocks' sums of up to MT_BLK blocks wait there
  * for one thread to add them in order.  Bound by the exponentials.  200 pairs of
- * 1,337 rows with up to 3,000 columns: 6.9 ms before */
+ * 1,337 rows with up to 3,000 columns: 6.9 -> 1.33 ms */
 constexpr int MT_BLK = 2048;
 template <int R>
 __global__ __launch_bounds__(1024) void k_map_total(ScoreCtx c, MapArgs m)

@@ -343,8 +343,8 @@ int  cbp_score_block(cbp_handle* h, int32_t qidx, int32_t pronr, float* S, float
  * one GPU: calls that overlap on one GPU (two threads or two handles) race */
 int  cbp_phase1_keys_noalloc(cbp_handle* h, int32_t qidx, uint64_t* keys /* [nprof] */);
 
-/* tuning of the phase-1 launch geometry: target DB columns per wave segment
- * (>= 64), maximum query rows per lane (1..5) and waves per workgroup
+/* tuning of the phase-1 launch geometry: most DB columns per wave segment
+ * (>= 64; smaller chunks are cut finer to fill the GPU), maximum query rows per lane (1..5) and waves per workgroup
  * (1, 2, 4, 8); no reference counterpart (the reference fixes 32x32 blocks,
  * cudp/CuBatchDP_com.h:16-30) */
 int  cbp_set_tuning(cbp_handle* h, int32_t seg_cols, int32_t rmax, int32_t nw);
@@ -394,13 +394,14 @@ int  cbp_set_mfma(cbp_handle* h, int32_t on);
  * group at most rmax query rows per lane and as few stripes (waves per pair)
  * as that allows, so each wave works on more rows and fewer waves wait at
  * the band's per-step barriers; rmax = 0 keeps the long pairs' geometry
- * (one band of up to 8 waves, R = ceil(Lq/512)) for every pair.  Results are
+ * (one row per lane in up to 16 waves for queries of at most 1,024 positions,
+ * else up to 8 waves of R = ceil(Lq/512)) for every pair.  Results are
  * bit-identical either way.  Replaces the fixed 32x32-block schedule of
  * ExecMAPDP_Parent_DynPlm (cumapdp/CuBatchMAPDP_prnt.cu:18-115) */
 int  cbp_set_map_rows(cbp_handle* h, int32_t rmax);
 
 /* MAP forward and backward passes (on = 1, the default): for queries whose
- * stripes fit one band of 8 waves, persistent workgroups stream their pairs
+ * stripes fit one band (16 waves at one row per lane, else 8), persistent workgroups stream their pairs
  * through the band back to back, so waves do not idle while a pair's band
  * fills and drains; on = 0 runs one workgroup per pair.  Results are
  * bit-identical either way.  Replaces the per-pair launch loops of
