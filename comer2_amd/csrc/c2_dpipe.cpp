@@ -169,7 +169,8 @@ int dl_chain(cbp_handle* h, int i, const DlPlan& P)
     DCHK(c2_launch_zero_u32((uint32_t*)q.cnt.p, DL_NCNT, st));
     DCHK(c2_dl_candidates(w.dk, d.nprof, w.scorethld, b, d.len.as<int32_t>(), hp.nstripes, q.dargs.as<P1Args>(),
                           q.tiles.as<P1Tile>(), 0, q.ntiles.as<int32_t>(), st));
-    /* the backtrack pass: the query's candidates in pairs from its queue */
+    /* the backtrack pass: the query's candidates from its queue, in pairs, or
+     * one by one when a candidate's stripes run in a band of waves */
     P1QueueArgs qa;
     qa.args = q.dargs.as<P1Args>();
     qa.tiles = q.tiles.as<P1Tile>();
@@ -191,7 +192,8 @@ int dl_chain(cbp_handle* h, int i, const DlPlan& P)
                             q.cnt.as<int32_t>() + DL_NC));
         DCHK(hipEventRecord(h->gjoin[0], h->xstream[0]));
     }
-    DCHK(c2_launch_phase1q(qa, hp.R, 2, true, P.grid[i], P.lds[i], st));
+    if (hp.nstripes > 1) DCHK(c2_launch_btck_band(qa, hp.R, hp.nstripes, P.grid[i], st));
+    else DCHK(c2_launch_phase1q(qa, hp.R, 2, true, P.grid[i], P.lds[i], st));
     DCHK(c2_launch_finalize(sc, sl.cand.as<int32_t>(), k.capC, w.dk, sl.btck.as<uint32_t>(), sl.off.as<int64_t>(),
                             sl.fin.as<FinRec>(), st, q.cnt.as<int32_t>() + DL_NC));
     DCHK(c2_dl_pass(sl.fin.as<FinRec>(), sl.cand.as<int32_t>(), d.len.as<int32_t>(), d.eno.as<float>(),
@@ -373,9 +375,9 @@ int c2_run_queries_dev(cbp_handle* h, const int32_t* qidx, int32_t nq, const flo
         const size_t lds = c2_phase1_lds_bytes(hp.R, 2, hp.nstripes);
         if (lds > 80 * 1024) return c2_fail(h, CBP_ERR_STATE, "backtrack pass exceeds the LDS");
         P.lds[i] = lds;
-        P.grid[i] = c2_phase1q_grid(hp.R, 2, true, lds);
+        P.grid[i] = hp.nstripes > 1 ? c2_btck_band_grid(hp.R, hp.nstripes) : c2_phase1q_grid(hp.R, 2, true, lds);
         if (P.grid[i] < 1) return c2_fail(h, CBP_ERR_HIP, "backtrack queue occupancy");
-        if (hp.nstripes > 1) botw = std::max<int64_t>(botw, (int64_t)P.grid[i] * 2 * 5 * h->chunk_maxlen);
+        if (hp.nstripes > 1) botw = std::max<int64_t>(botw, (int64_t)P.grid[i] * 5 * h->chunk_maxlen);
         uint64_t delta = 0;
         w.sspace = c2_length_adjustment(h->opt, (uint64_t)hp.Lq, dblen, nseqs, &delta);
         StatParams& sp = P.sp[i];

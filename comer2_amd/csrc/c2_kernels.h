@@ -244,6 +244,11 @@ hipError_t c2_launch_phase1(const P1Args& a, int R, int NW, bool btck, hipStream
 int c2_phase1q_grid(int R, int NW, bool btck, size_t lds, bool mf = false);
 hipError_t c2_launch_phase1q(const P1QueueArgs& q, int R, int NW, bool btck, int grid, size_t lds, hipStream_t stream,
                              bool mf = false);
+/* the backtrack pass of a query of two or more stripes, one candidate per
+ * workgroup and a stripe per wave: qa.args one query's, no tiles, qa.botw
+ * [grid][5][bot_ld] */
+int c2_btck_band_grid(int R, int nstripes);
+hipError_t c2_launch_btck_band(const P1QueueArgs& q, int R, int nstripes, int grid, hipStream_t stream);
 
 constexpr int C2_SDP_BAND = 4;      /* waves of a soft-DP workgroup, one stripe each */
 /* soft DP: one pair of (query, chunk profile) and its workspace offsets (floats) */

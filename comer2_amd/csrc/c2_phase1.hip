@@ -51,6 +51,21 @@ constexpr int NS_BASE = 35, NS_TOP = 39;   /* slot stride without / with the str
 constexpr int F_CV = 39, F_CVP = 58, F_CVA = 59, NS_CV = 61;
 constexpr int CV_MAP = 128;                /* LDS words for the CV map */
 
+/* a band of waves over one candidate's stripes (k_btck_band): wave w takes
+ * stripes w, w + nw, ...; stripe s starts at the workgroup's barrier
+ * (s / nw) * period + BAND_LAG * (s % nw), where the waves hand their last rows
+ * over in rings of HAND columns in LDS */
+constexpr int BAND_MAX = 4, BAND_LAG = 3, HAND = 64;
+struct P1Band {
+    int nw;                 /* waves of the workgroup */
+    int period;             /* barriers from a round of nw stripes to the next */
+    int cut;                /* columns of the candidate to sweep */
+    float* hout;            /* [5][HAND] the wave's last row */
+    const float* hin;       /* the wave before's */
+    int g;                  /* barriers passed */
+    __device__ __forceinline__ void sync() { __syncthreads(); g++; }
+};
+
 /* tops: the ring carries the stripe's top boundary; rtop: read it from the
  * hand-off buffer (stripes after the first) instead of the zero row -1 */
 /* the profile of the column lane loads in the refill of block t0 (loaded
@@ -62,10 +77,11 @@ __device__ __forceinline__ int block_profile(PA& a, int lane, int t0, int64_t c_
     return (lane < BK && c < c_end) ? a.addrpro[c] : -1;
 }
 
-template <int R, bool CV, int BK, class PA>
+template <int R, bool CV, int BK, bool HANDIN = false, class PA>
 __device__ __forceinline__ void load_block(PA& a, float* ring, int ns, int lane, int t0,
                                            int64_t c_begin, int64_t c_end, bool tops, bool rtop, int p,
-                                           const float* bot, int64_t bld, int64_t bc0)
+                                           const float* bot, int64_t bld, int64_t bc0,
+                                           const float* hin = nullptr)
 {
     if (lane >= BK) return;
     float* rc = ring + ((t0 + lane) % RING) * ns;
@@ -110,7 +126,10 @@ __device__ __forceinline__ void load_block(PA& a, float* ring, int ns, int lane,
         const uint32_t bins = (uint32_t)(int)(sp[0] * 9.999f) | ((uint32_t)(int)(sp[(size_t)npos] * 9.999f) << 4) |
                               ((uint32_t)(int)(sp[2 * (size_t)npos] * 9.999f) << 8);
         rc[F_BIN] = __uint_as_float(bins);
-        if (tops) {
+        if (HANDIN && rtop && hin) {
+            const float* bt = hin + ((t0 + lane) & (HAND - 1));
+            for (int s = 0; s < 5; s++) rc[F_TOP + s] = bt[s * HAND];
+        } else if (tops) {
             const float* bt = bot + (c - bc0);
             for (int s = 0; s < 5; s++)
                 rc[F_TOP + s] = rtop ? bt[(size_t)s * bld] : 0.0f;
@@ -155,10 +174,12 @@ typedef const __attribute__((address_space(4))) P1Args CP1Args;
  * botw != nullptr: the stripe hand-off goes to the wave's own scratch rows
  * of bot_ld columns (indexed from the segment's first column) instead of the
  * query's per-column buffer a.bot */
-template <int R, int NW, bool BTCK, bool CV, bool MF, class PA>
-__device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw, int64_t bot_ld)
+template <int R, int NW, bool BTCK, bool CV, bool MF, class PA, bool BAND = false>
+__device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw, int64_t bot_ld,
+                                         P1Band* bd = nullptr)
 {
     static_assert(!(MF && CV), "the matrix-core contraction has no context-vector form");
+    static_assert(!BAND || (BTCK && !CV && !MF), "a band sweeps one candidate for its backtrack codes");
     /* refill: BK columns, LEAD steps ahead of the column that starts the
      * block.  The matrix-core form reads columns up to 3 ahead of lane 0 at
      * every fourth step, so it refills 16 columns 4 steps ahead (the ring
@@ -173,7 +194,8 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
     const bool tops = a.nstripes > 1;
     const int ns = CV ? NS_CV : (tops ? NS_TOP : NS_BASE);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-    float* ring = sLD + 5 * SL + (size_t)wv * ns * RING;
+    /* a band's waves are on different stripes: their tables stay in memory */
+    float* ring = (BAND ? lds : sLD + 5 * SL) + (size_t)wv * ns * RING;
     /* the CV map after the rings */
     float* sMap = sLD + 5 * SL + (size_t)NW * ns * RING;
     if constexpr (CV) {
@@ -181,23 +203,27 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
             sMap[i] = i < a.cvs.card ? a.cvs.map[i] : 0.0f;
     }
 
-    for (int s = 0; s < a.nstripes; s++) {
+    const int s0 = BAND ? wv : 0, sinc = BAND ? bd->nw : 1;
+    for (int s = s0; s < a.nstripes; s += sinc) {
         const int rbase = s * SL;
-        __syncthreads();
-        for (int i = threadIdx.x; i < 30 * SL; i += 64 * NW)
-            sQT[i] = a.QT[(size_t)(i / SL) * a.Lpad + rbase + (i % SL)];
-        for (int i = threadIdx.x; i < 5 * SL; i += 64 * NW) {
-            sLL[i] = a.lleft[(size_t)(i / SL) * a.Lpad + rbase + (i % SL)];
-            sLD[i] = a.ldiag[(size_t)(i / SL) * a.Lpad + rbase + (i % SL)];
+        if constexpr (!BAND) {
+            __syncthreads();
+            for (int i = threadIdx.x; i < 30 * SL; i += 64 * NW)
+                sQT[i] = a.QT[(size_t)(i / SL) * a.Lpad + rbase + (i % SL)];
+            for (int i = threadIdx.x; i < 5 * SL; i += 64 * NW) {
+                sLL[i] = a.lleft[(size_t)(i / SL) * a.Lpad + rbase + (i % SL)];
+                sLD[i] = a.ldiag[(size_t)(i / SL) * a.Lpad + rbase + (i % SL)];
+            }
+            __syncthreads();
+            if (seg >= a.nseg) continue;
         }
-        __syncthreads();
-        if (seg >= a.nseg) continue;
 
         const int pb = a.seg_pb[seg], pe = a.seg_pe[seg];
         const int64_t c_begin = a.dist[pb];
         const int64_t c_full = (int64_t)a.dist[pe - 1] + a.len[pe - 1];
         int64_t c_end = c_full;
-        if (BTCK) {
+        if constexpr (BAND) c_end = c_begin + bd->cut;
+        else if (BTCK) {
             /* one candidate profile: the backtrace starts at the maximum's
              * column x (the key phase 1 left), so columns past x are not swept;
              * the codes keep the whole profile's stride */
@@ -257,8 +283,15 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
             }
         }
         wave_lds_sync();
+        /* the row above comes from the wave before, at a round's first stripe
+         * from the workgroup's hand-off row in memory */
+        const float* hin = BAND && wv > 0 ? bd->hin : nullptr;
+        if constexpr (BAND) {
+            const int gs = (s / bd->nw) * bd->period + BAND_LAG * wv;
+            while (bd->g <= gs) bd->sync();
+        }
         int pn = block_profile<BK>(a, lane, 0, c_begin, c_end);
-        load_block<R, CV, BK>(a, ring, ns, lane, 0, c_begin, c_end, tops, s > 0, pn, bot, bld, bc0);
+        load_block<R, CV, BK, BAND>(a, ring, ns, lane, 0, c_begin, c_end, tops, s > 0, pn, bot, bld, bc0, hin);
         wave_lds_sync();
 
         S5 H[R];
@@ -312,6 +345,19 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
                 for (int i = 0; i < 19; i++) dc[i] = rs[F_CV + i];
                 dpr = rs[F_CVP];
                 dna = rs[F_CVA];
+            }
+        };
+        /* a band's SS-table terms of the next step, read from memory a step ahead */
+        float tq[BAND ? 3 : 1][BAND ? R : 1];
+        const float* QTs = a.QT + rbase + R * lane;
+        auto read_qt = [&]() {
+            if constexpr (BAND) {
+#pragma unroll
+                for (int j = 0; j < 3; j++) {
+                    const float* p = QTs + (size_t)((uint32_t)(10 * j) + ((bb >> (4 * j)) & 15u)) * a.Lpad;
+#pragma unroll
+                    for (int k = 0; k < R; k++) tq[j][k] = p[k];
+                }
             }
         };
         /* matrix-core form: at every fourth step t = 4s each group of four
@@ -377,6 +423,7 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
             }
         };
         read_col();
+        read_qt();
         for (int t = 0; t < nsteps; t++) {
             /* profile start: flush, reset to the column -1 boundary */
             const bool first = (xloc == 0);
@@ -399,13 +446,25 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
 #pragma unroll
                     for (int k = 0; k < R; k++) {
                         const int sl = R * lane + k;
+                        if constexpr (BAND) {
+                            const float* g = a.lleft + rbase + sl;
+                            H[k].mm = g[0]; H[k].mi = g[(size_t)a.Lpad]; H[k].im = g[2 * (size_t)a.Lpad];
+                            H[k].dn = g[3 * (size_t)a.Lpad]; H[k].nd = g[4 * (size_t)a.Lpad];
+                            continue;
+                        }
                         H[k].mm = sLL[0 * SL + sl]; H[k].mi = sLL[1 * SL + sl];
                         H[k].im = sLL[2 * SL + sl]; H[k].dn = sLL[3 * SL + sl];
                         H[k].nd = sLL[4 * SL + sl];
                     }
                     const int sl0 = R * lane;
+                    if constexpr (BAND) {
+                        const float* g = a.ldiag + rbase + sl0;
+                        D.mm = g[0]; D.mi = g[(size_t)a.Lpad]; D.im = g[2 * (size_t)a.Lpad];
+                        D.dn = g[3 * (size_t)a.Lpad]; D.nd = g[4 * (size_t)a.Lpad];
+                    } else {
                     D.mm = sLD[0 * SL + sl0]; D.mi = sLD[1 * SL + sl0]; D.im = sLD[2 * SL + sl0];
                     D.dn = sLD[3 * SL + sl0]; D.nd = sLD[4 * SL + sl0];
+                    }
                 }
 #pragma unroll
                 for (int k = 1; k < R; k++)
@@ -448,7 +507,8 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
                 float t0[R], t1[R], t2[R];
 #pragma unroll
                 for (int k = 0; k < R; k++) {
-                    t0[k] = sQT[co[0] + k]; t1[k] = sQT[co[1] + k]; t2[k] = sQT[co[2] + k];
+                    if constexpr (BAND) { t0[k] = tq[0][k]; t1[k] = tq[1][k]; t2[k] = tq[2][k]; }
+                    else { t0[k] = sQT[co[0] + k]; t1[k] = sQT[co[1] + k]; t2[k] = sQT[co[2] + k]; }
                 }
 #pragma unroll
                 for (int k = 0; k < R; k++) {
@@ -524,7 +584,11 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
             }
             if (BTCK) btw[(size_t)t * 64 + lane] = bw;
             if (wbot && t >= 63 && t - 63 < ncols) {
-                if (lane == 63) {
+                if (BAND && lane == 63 && wv + 1 < bd->nw) {
+                    float* bt = bd->hout + ((t - 63) & (HAND - 1));
+                    bt[0 * HAND] = H[R - 1].mm; bt[1 * HAND] = H[R - 1].mi; bt[2 * HAND] = H[R - 1].im;
+                    bt[3 * HAND] = H[R - 1].dn; bt[4 * HAND] = H[R - 1].nd;
+                } else if (lane == 63) {
                     float* bt = bot + ((c_begin + t - 63) - bc0);
                     bt[0 * (size_t)bld] = H[R - 1].mm; bt[1 * (size_t)bld] = H[R - 1].mi;
                     bt[2 * (size_t)bld] = H[R - 1].im; bt[3 * (size_t)bld] = H[R - 1].dn;
@@ -551,17 +615,26 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
             /* the block after next: its first column is the top boundary the
              * next step reads ahead of its rows */
             if (((t + LEAD) % BK) == 0) {
-                load_block<R, CV, BK>(a, ring, ns, lane, t + LEAD, c_begin, c_end, tops, s > 0,
-                                      block_profile<BK>(a, lane, t + LEAD, c_begin, c_end), bot, bld, bc0);
+                if constexpr (BAND) bd->sync();
+                load_block<R, CV, BK, BAND>(a, ring, ns, lane, t + LEAD, c_begin, c_end, tops, s > 0,
+                                            block_profile<BK>(a, lane, t + LEAD, c_begin, c_end), bot, bld, bc0,
+                                            hin);
                 wave_lds_sync();
             }
             read_col();
+            read_qt();
         }
         if (curpid >= 0 && best > 0.0f) {
             const int tb = bpos >> 3, kb = bpos & 7;
             atomicMax(a.keys + curpid, mkkey(best, (tb - lane) - pstart, y0 + kb));
         }
-        if (tops) __threadfence();
+        if (tops && !BAND) __threadfence();
+    }
+    if constexpr (BAND) {
+        /* to the barrier after the last stripe's last block, every wave alike */
+        const int sl = a.nstripes - 1, nsteps = bd->cut + 63;
+        const int end = (sl / bd->nw) * bd->period + BAND_LAG * (sl % bd->nw) + (nsteps + LEAD - 1) / BK + 1;
+        while (bd->g <= end) bd->sync();
     }
 }
 
@@ -598,6 +671,58 @@ __global__ __launch_bounds__(64 * NW, 1) void k_phase1q(P1QueueArgs qa)
          * constant address space, as kernel arguments are */
         CP1Args* ap = (CP1Args*)(qa.args + tq);
         p1_sweep<R, NW, BTCK, false, MF, CP1Args>(*ap, tg * NW + wv, lds, botw, qa.bot_ld);
+    }
+}
+
+/* the backtrack pass of a query of several stripes: a workgroup takes a
+ * candidate and its waves sweep the stripes side by side instead of one wave
+ * one after another.  With steps t = 0.. of a stripe, its refill of columns
+ * 32k.. (just before step 32k - 1) follows barrier G + k, G the stripe's first;
+ * the wave before has then finished its step 32k + 94, which completes the
+ * last row of those columns, and has not reached the step that takes their
+ * slots in its ring of 64.  A round of nw stripes starts when wave 0 is done
+ * with the round before (period: its blocks, at least 3 nw), and its first
+ * stripe reads the last wave's row, kept in memory, three blocks behind it.
+ * Up to BAND_MAX waves: 15 KB of LDS each, so several workgroups share a CU
+ * and a list of many short candidates keeps the CU as busy as before; the
+ * stripes are dealt evenly to the rounds (6: 3 and 3).  Bound by the longest
+ * candidate's chain of steps.  1,337 rows in 6 stripes, candidates of up to
+ * 3,000 columns: 12.8 ms one wave at a time, 5.15 ms in bands of 3. */
+template <int R>
+__global__ __launch_bounds__(64 * BAND_MAX, 2) void k_btck_band(P1QueueArgs qa)
+{
+    extern __shared__ float lds[];
+    __shared__ int tile_s, cut_s;
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    CP1Args* ap = (CP1Args*)qa.args;
+    const int nw = (int)(blockDim.x >> 6), nseg = ap->nseg;
+    float* hand = lds + (size_t)nw * NS_TOP * RING;
+    float* botw = qa.botw + (size_t)blockIdx.x * 5 * qa.bot_ld;
+    P1Band bd;
+    bd.nw = nw;
+    bd.hout = hand + wv * 5 * HAND;
+    bd.hin = hand + (wv > 0 ? wv - 1 : 0) * 5 * HAND;
+    for (;;) {
+        if (threadIdx.x == 0) {
+            const int ti = (int)atomicAdd(qa.head, 1u);
+            tile_s = ti;
+            if (ti < nseg) {
+                /* the columns up to the maximum's (the key phase 1 left) */
+                const int pb = ap->seg_pb[ti];
+                const uint32_t xy = 0xFFFFFFFFu - (uint32_t)ap->keys[pb];
+                const int len = ap->len[pb], cut = (int)(xy >> 16) + 1;
+                cut_s = cut < len ? cut : len;
+            }
+        }
+        __syncthreads();
+        const int ti = __builtin_amdgcn_readfirstlane(tile_s);
+        if (ti >= nseg) break;
+        bd.cut = __builtin_amdgcn_readfirstlane(cut_s);
+        const int blocks = (bd.cut + 63 + 1) / BLK + 1;
+        bd.period = blocks > BAND_LAG * nw ? blocks : BAND_LAG * nw;
+        bd.g = 0;
+        p1_sweep<R, BAND_MAX, true, false, false, CP1Args, true>(*ap, ti, lds, botw, qa.bot_ld, &bd);
+        __syncthreads();
     }
 }
 
@@ -779,11 +904,29 @@ static const void* phase1q_fn(int R, int NW, bool btck, bool mf)
     return nullptr;
 }
 
-int c2_phase1q_grid(int R, int NW, bool btck, size_t lds, bool mf)
+static const void* btck_band_fn(int R)
 {
-    const void* fn = phase1q_fn(R, NW, btck, mf);
+    switch (R) {
+        case 1: return (const void*)k_btck_band<1>;
+        case 2: return (const void*)k_btck_band<2>;
+        case 3: return (const void*)k_btck_band<3>;
+        case 4: return (const void*)k_btck_band<4>;
+        case 5: return (const void*)k_btck_band<5>;
+        default: return nullptr;
+    }
+}
+
+int c2_btck_band_waves(int nstripes)
+{
+    const int rounds = (nstripes + BAND_MAX - 1) / BAND_MAX;
+    return (nstripes + rounds - 1) / rounds;
+}
+
+size_t c2_btck_band_lds_bytes(int nw) { return sizeof(float) * (size_t)nw * (NS_TOP * RING + 5 * HAND); }
+
+static int resident_grid(const void* fn, int NW, size_t lds)
+{
     if (!fn || lds > Q_MAX_DYN_LDS) return 0;
-    /* the kernel's own pull slot is static LDS: the dynamic limit stays below 160 KiB */
     if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, (int)Q_MAX_DYN_LDS) != hipSuccess) return 0;
     int dev = 0, ncu = 0, per = 0;
     if (hipGetDevice(&dev) != hipSuccess ||
@@ -795,6 +938,28 @@ int c2_phase1q_grid(int R, int NW, bool btck, size_t lds, bool mf)
         if (per < 1) per = 1;
     }
     return per * ncu;
+}
+
+int c2_btck_band_grid(int R, int nstripes)
+{
+    const int nw = c2_btck_band_waves(nstripes);
+    return resident_grid(btck_band_fn(R), nw, c2_btck_band_lds_bytes(nw));
+}
+
+hipError_t c2_launch_btck_band(const P1QueueArgs& q, int R, int nstripes, int grid, hipStream_t stream)
+{
+    const void* fn = btck_band_fn(R);
+    const int nw = c2_btck_band_waves(nstripes);
+    if (!fn || grid < 1 || nstripes < 2 || !q.botw) return hipErrorInvalidValue;
+    P1QueueArgs qa = q;
+    void* args[] = {&qa};
+    return hipLaunchKernel(fn, dim3((unsigned)grid), dim3(64 * nw), args, c2_btck_band_lds_bytes(nw), stream);
+}
+
+int c2_phase1q_grid(int R, int NW, bool btck, size_t lds, bool mf)
+{
+    /* the kernel's own pull slot is static LDS: the dynamic limit stays below 160 KiB */
+    return resident_grid(phase1q_fn(R, NW, btck, mf), NW, lds);
 }
 
 hipError_t c2_launch_phase1q(const P1QueueArgs& q, int R, int NW, bool btck, int grid, size_t lds, hipStream_t stream,
