@@ -44,6 +44,8 @@ struct P1Args {
     const int32_t* seg_pb; /* [nseg] first profile of each segment */
     const int32_t* seg_pe; /* [nseg] one past the last profile */
     int32_t nseg;
+    int32_t nlong;        /* of these, the leading ones worth a workgroup each (DB sweep of one query) */
+    int32_t bstripes, bwaves;   /* set by the launch: a long segment's stripes and the waves that take them */
     int32_t mfma;         /* the DB sweep forms the 20-term sums on the matrix cores */
     /* outputs */
     unsigned long long* keys;   /* [nprof] */

@@ -315,6 +315,17 @@ static int build_segset(cbp_handle* h, const cbp_profiles* s, int64_t target, Se
     std::stable_sort(v.begin(), v.end(), [&](const auto& x, const auto& y) { return cols(x) > cols(y); });
     g->nseg = (int32_t)v.size();
     g->maxcols = (int32_t)cols(v[0]);
+    /* a segment of more than twice the target is a long profile that ends
+     * after the rest (which is two segments per slot): it goes to a workgroup
+     * of its own, at most a quarter of the device.  More than 1.5 times the
+     * target, or half the device, takes CUs from the rest (15,000 profiles x
+     * 223 rows: 3.35 ms without, 3.05 so, 3.99 at 1.5; 60,000 x 300: 14.9,
+     * 14.9 and 18.2 at 1.2), three times leaves some behind (1,337 rows: 21.6,
+     * 15.9 and 16.6 ms).  Up to two segments per CU no wave waits for its
+     * workgroup's others, and a band is no faster (0.36 against 0.40 ms) */
+    g->nlong = 0;
+    if (g->nseg > 2 * h->ncu)
+        while (g->nlong < h->ncu / 4 && cols(v[g->nlong]) > 2 * target) g->nlong++;
     g->b.resize(v.size()); g->e.resize(v.size());
     for (size_t i = 0; i < v.size(); i++) { g->b[i] = v[i].first; g->e[i] = v[i].second; }
     int rc;
@@ -520,7 +531,7 @@ int c2_fill_p1args(cbp_handle* h, DevQuery* dq, P1Args* a)
     a->ssswgt = h->opt.ssswgt;
     c2_fill_cvs(h, dq, &a->cvs);
     const SegSet& g = *h->segs[0];
-    a->seg_pb = g.db.as<int32_t>(); a->seg_pe = g.de.as<int32_t>(); a->nseg = g.nseg;
+    a->seg_pb = g.db.as<int32_t>(); a->seg_pe = g.de.as<int32_t>(); a->nseg = g.nseg; a->nlong = g.nlong;
     a->mfma = h->use_mfma;
     return CBP_OK;
 }

@@ -108,7 +108,7 @@ extern "C" int cbp_phase1_keys_noalloc(cbp_handle* h, int32_t qidx, uint64_t* ke
     a.shift = h->opt.mapaln ? 0.002f : 0.0003f;
     a.ssswgt = h->opt.ssswgt;
     const SegSet& g = *h->segs[0];
-    a.seg_pb = g.db.as<int32_t>(); a.seg_pe = g.de.as<int32_t>(); a.nseg = g.nseg;
+    a.seg_pb = g.db.as<int32_t>(); a.seg_pe = g.de.as<int32_t>(); a.nseg = g.nseg; a.nlong = g.nlong;
     a.keys = (unsigned long long*)(base + o_keys);
     a.bot = hp.nstripes > 1 ? (float*)(base + o_bot) : nullptr;
     const int nw = c2_phase1_waves(h, hp.R, hp.nstripes, a.nseg);

@@ -51,18 +51,25 @@ constexpr int NS_BASE = 35, NS_TOP = 39;   /* slot stride without / with the str
 constexpr int F_CV = 39, F_CVP = 58, F_CVA = 59, NS_CV = 61;
 constexpr int CV_MAP = 128;                /* LDS words for the CV map */
 
-/* a band of waves over one candidate's stripes (k_btck_band): wave w takes
+/* a band of waves over one segment's stripes (k_btck_band, k_phase1_mix): wave w takes
  * stripes w, w + nw, ...; stripe s starts at the workgroup's barrier
  * (s / nw) * period + BAND_LAG * (s % nw), where the waves hand their last rows
  * over in rings of HAND columns in LDS */
 constexpr int BAND_MAX = 4, BAND_LAG = 3, HAND = 64;
 struct P1Band {
-    int nw;                 /* waves of the workgroup */
+    int ns;                 /* stripes */
+    int nw;                 /* waves of the band; others only meet the barriers */
     int period;             /* barriers from a round of nw stripes to the next */
-    int cut;                /* columns of the candidate to sweep */
+    int cut;                /* columns to sweep */
     float* hout;            /* [5][HAND] the wave's last row */
     const float* hin;       /* the wave before's */
     int g;                  /* barriers passed */
+    __device__ __forceinline__ void start()
+    {
+        const int blocks = (cut + 63 + 1) / BLK + 1;
+        period = blocks > BAND_LAG * nw ? blocks : BAND_LAG * nw;
+        g = 0;
+    }
     __device__ __forceinline__ void sync() { __syncthreads(); g++; }
 };
 
@@ -179,7 +186,7 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
                                          P1Band* bd = nullptr)
 {
     static_assert(!(MF && CV), "the matrix-core contraction has no context-vector form");
-    static_assert(!BAND || (BTCK && !CV && !MF), "a band sweeps one candidate for its backtrack codes");
+    static_assert(!(MF && BAND), "the matrix-core contraction has no band form");
     /* refill: BK columns, LEAD steps ahead of the column that starts the
      * block.  The matrix-core form reads columns up to 3 ahead of lane 0 at
      * every fourth step, so it refills 16 columns 4 steps ahead (the ring
@@ -191,20 +198,22 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
     float* sQT = lds;                           /* [30][SL] */
     float* sLL = sQT + 30 * SL;                 /* [5][SL] */
     float* sLD = sLL + 5 * SL;                  /* [5][SL] */
-    const bool tops = a.nstripes > 1;
+    int nst = a.nstripes;
+    if constexpr (BAND) nst = bd->ns;
+    const bool tops = nst > 1;
     const int ns = CV ? NS_CV : (tops ? NS_TOP : NS_BASE);
     const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
     /* a band's waves are on different stripes: their tables stay in memory */
     float* ring = (BAND ? lds : sLD + 5 * SL) + (size_t)wv * ns * RING;
     /* the CV map after the rings */
-    float* sMap = sLD + 5 * SL + (size_t)NW * ns * RING;
+    float* sMap = BAND ? lds + (size_t)bd->nw * (ns * RING + 5 * HAND) : sLD + 5 * SL + (size_t)NW * ns * RING;
     if constexpr (CV) {
-        for (int i = threadIdx.x; i < CV_MAP; i += 64 * NW)
+        for (int i = threadIdx.x; i < CV_MAP; i += BAND ? (int)blockDim.x : 64 * NW)
             sMap[i] = i < a.cvs.card ? a.cvs.map[i] : 0.0f;
     }
 
-    const int s0 = BAND ? wv : 0, sinc = BAND ? bd->nw : 1;
-    for (int s = s0; s < a.nstripes; s += sinc) {
+    const int s0 = BAND ? (wv < bd->nw ? wv : nst) : 0, sinc = BAND ? bd->nw : 1;
+    for (int s = s0; s < nst; s += sinc) {
         const int rbase = s * SL;
         if constexpr (!BAND) {
             __syncthreads();
@@ -305,7 +314,7 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
         }
         float best = 0.0f;
         int bpos = 0, curpid = -1, pstart = 0, cA = 0, cW = 0;
-        const bool wbot = tops && (s + 1 < a.nstripes);
+        const bool wbot = tops && (s + 1 < nst);
         uint32_t* btw = nullptr;
         if (BTCK) btw = a.btck + a.btck_off[seg] + (size_t)s * bstride * 64;
 
@@ -632,7 +641,7 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
     }
     if constexpr (BAND) {
         /* to the barrier after the last stripe's last block, every wave alike */
-        const int sl = a.nstripes - 1, nsteps = bd->cut + 63;
+        const int sl = nst - 1, nsteps = bd->cut + 63;
         const int end = (sl / bd->nw) * bd->period + BAND_LAG * (sl % bd->nw) + (nsteps + LEAD - 1) / BK + 1;
         while (bd->g <= end) bd->sync();
     }
@@ -674,6 +683,37 @@ __global__ __launch_bounds__(64 * NW, 1) void k_phase1q(P1QueueArgs qa)
     }
 }
 
+/* a query's sweep where single segments are long beside the rest (the first
+ * a.nlong of the list, widest first): the first nlong workgroups sweep one of
+ * these each, RB rows per lane, their stripes side by side in a.bwaves waves
+ * (k_btck_band explains the schedule), the others NW segments as k_phase1
+ * does.  RB is 1 for a query of one stripe, which is cut for this, else R.
+ * The SS table of a band comes from memory, which is why the rest, that fills
+ * the chip, keeps its shared copy in LDS.  Without the bands a profile of
+ * 3,000 columns against 1,337 rows was 6 stripes x 3,063 steps in one wave,
+ * two waves on each SIMD: 12,000 profiles took 21.6 ms, now 15.9; with
+ * context vectors, 181 rows x 6,000: 1.97 -> 1.65; 150 x 2,000: 0.88 -> 0.76 ms. */
+template <int R, int RB, int NW, bool CV>
+__global__ __launch_bounds__(64 * NW, 1) void k_phase1_mix(P1Args a)
+{
+    extern __shared__ float lds[];
+    const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int b = (int)blockIdx.x;
+    if (b >= a.nlong) {
+        p1_sweep<R, NW, false, CV, false, const P1Args>(a, a.nlong + (b - a.nlong) * NW + wv, lds, nullptr, 0);
+        return;
+    }
+    P1Band bd;
+    bd.ns = a.bstripes; bd.nw = a.bwaves;
+    float* hand = lds + (size_t)bd.nw * (CV ? NS_CV : NS_TOP) * RING;
+    bd.hout = hand + wv * 5 * HAND;
+    bd.hin = hand + (wv > 0 ? wv - 1 : 0) * 5 * HAND;
+    const int pb = a.seg_pb[b], pe = a.seg_pe[b];
+    bd.cut = __builtin_amdgcn_readfirstlane((int)((int64_t)a.dist[pe - 1] + a.len[pe - 1] - (int64_t)a.dist[pb]));
+    bd.start();
+    p1_sweep<RB, NW, false, CV, false, const P1Args, true>(a, b, lds, nullptr, 0, &bd);
+}
+
 /* the backtrack pass of a query of several stripes: a workgroup takes a
  * candidate and its waves sweep the stripes side by side instead of one wave
  * one after another.  With steps t = 0.. of a stripe, its refill of columns
@@ -699,7 +739,7 @@ __global__ __launch_bounds__(64 * BAND_MAX, 2) void k_btck_band(P1QueueArgs qa)
     float* hand = lds + (size_t)nw * NS_TOP * RING;
     float* botw = qa.botw + (size_t)blockIdx.x * 5 * qa.bot_ld;
     P1Band bd;
-    bd.nw = nw;
+    bd.nw = nw; bd.ns = ap->nstripes;
     bd.hout = hand + wv * 5 * HAND;
     bd.hin = hand + (wv > 0 ? wv - 1 : 0) * 5 * HAND;
     for (;;) {
@@ -718,9 +758,7 @@ __global__ __launch_bounds__(64 * BAND_MAX, 2) void k_btck_band(P1QueueArgs qa)
         const int ti = __builtin_amdgcn_readfirstlane(tile_s);
         if (ti >= nseg) break;
         bd.cut = __builtin_amdgcn_readfirstlane(cut_s);
-        const int blocks = (bd.cut + 63 + 1) / BLK + 1;
-        bd.period = blocks > BAND_LAG * nw ? blocks : BAND_LAG * nw;
-        bd.g = 0;
+        bd.start();
         p1_sweep<R, BAND_MAX, true, false, false, CP1Args, true>(*ap, ti, lds, botw, qa.bot_ld, &bd);
         __syncthreads();
     }
@@ -845,14 +883,53 @@ static hipError_t launch_nw(const P1Args& a, int R, int grid, size_t lds, hipStr
     return hipGetLastError();
 }
 
+static const void* phase1_mix_fn(int R, bool multi, int NW, bool cv)
+{
+#define C2_P1M(RR)                                                                                       \
+    if (R == RR) {                                                                                       \
+        if (multi) return NW == 8 ? (const void*)k_phase1_mix<RR, RR, 8, false> : (const void*)k_phase1_mix<RR, RR, 4, false>; \
+        return NW == 8 ? (const void*)k_phase1_mix<RR, 1, 8, false> : (const void*)k_phase1_mix<RR, 1, 4, false>; \
+    }
+    if (cv) return R == 1 ? (const void*)k_phase1_mix<1, 1, 4, true> : (const void*)k_phase1_mix<2, 1, 4, true>;
+    C2_P1M(1) C2_P1M(2) C2_P1M(3) C2_P1M(4) C2_P1M(5)
+#undef C2_P1M
+    return nullptr;
+}
+
+/* the sweep with bands for the long segments; false: none here (no stripes to
+ * run side by side, or more than one round of them without a hand-off row) */
+static bool launch_mix(const P1Args& a0, int R, int NW, bool cv, size_t lds, hipStream_t stream, hipError_t* e)
+{
+    P1Args a = a0;
+    const bool multi = a.nstripes > 1;
+    if (a.nlong <= 0 || a.nlong > a.nseg || (NW != 8 && NW != 4)) return false;
+    const int rb = multi && !cv ? R : 1;
+    a.bstripes = (a.Lq + 64 * rb - 1) / (64 * rb);
+    if (a.bstripes < 2 || (!multi && a.bstripes > NW)) return false;
+    const void* fn = phase1_mix_fn(R, multi, NW, cv);
+    if (!fn) return false;
+    const int rounds = (a.bstripes + NW - 1) / NW;
+    a.bwaves = (a.bstripes + rounds - 1) / rounds;
+    const size_t bl = sizeof(float) * ((size_t)a.bwaves * ((cv ? NS_CV : NS_TOP) * RING + 5 * HAND) + (cv ? CV_MAP : 0));
+    const int grid = a.nlong + (a.nseg - a.nlong + NW - 1) / NW;
+    if (bl > lds) lds = bl;
+    void* args[] = {&a};
+    (void)hipGetLastError();   /* the status read after the launches is theirs alone */
+    *e = hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    if (*e == hipSuccess) *e = hipLaunchKernel(fn, dim3((unsigned)grid), dim3(64 * NW), args, lds, stream);
+    return true;
+}
+
 hipError_t c2_launch_phase1(const P1Args& a, int R, int NW, bool btck, hipStream_t stream)
 {
     if (a.nseg <= 0) return hipSuccess;
+    hipError_t e;
     if (a.cvs.wgt > 0.0f) {
         if (R < 1 || R > 2 || a.cvs.card < 1 || a.cvs.card > CV_MAP) return hipErrorInvalidValue;
         const int nw = btck ? 2 : 4;
         const int grid = (a.nseg + nw - 1) / nw;
         const size_t lds = phase1_cv_lds_bytes(R, nw);
+        if (!btck && launch_mix(a, R, nw, true, lds, stream, &e)) return e;
         if (btck) return R == 1 ? launch_cv<1, 2, true>(a, grid, lds, stream) : launch_cv<2, 2, true>(a, grid, lds, stream);
         return R == 1 ? launch_cv<1, 4, false>(a, grid, lds, stream) : launch_cv<2, 4, false>(a, grid, lds, stream);
     }
@@ -867,6 +944,7 @@ hipError_t c2_launch_phase1(const P1Args& a, int R, int NW, bool btck, hipStream
             default: return hipErrorInvalidValue;
         }
     }
+    if (!a.mfma && launch_mix(a, R, NW, false, lds, stream, &e)) return e;
     /* the DB sweep with the 20-term sums on the matrix cores */
     if (a.mfma) {
         switch (NW) {
