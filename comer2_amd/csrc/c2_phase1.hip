@@ -186,7 +186,7 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
                                          P1Band* bd = nullptr)
 {
     static_assert(!(MF && CV), "the matrix-core contraction has no context-vector form");
-    static_assert(!(MF && BAND), "the matrix-core contraction has no band form");
+    static_assert(!(BAND && (MF || CV)), "neither the matrix-core contraction nor the context vectors have a band form");
     /* refill: BK columns, LEAD steps ahead of the column that starts the
      * block.  The matrix-core form reads columns up to 3 ahead of lane 0 at
      * every fourth step, so it refills 16 columns 4 steps ahead (the ring
@@ -206,9 +206,9 @@ __device__ __forceinline__ void p1_sweep(PA& a, int seg, float* lds, float* botw
     /* a band's waves are on different stripes: their tables stay in memory */
     float* ring = (BAND ? lds : sLD + 5 * SL) + (size_t)wv * ns * RING;
     /* the CV map after the rings */
-    float* sMap = BAND ? lds + (size_t)bd->nw * (ns * RING + 5 * HAND) : sLD + 5 * SL + (size_t)NW * ns * RING;
+    float* sMap = sLD + 5 * SL + (size_t)NW * ns * RING;
     if constexpr (CV) {
-        for (int i = threadIdx.x; i < CV_MAP; i += BAND ? (int)blockDim.x : 64 * NW)
+        for (int i = threadIdx.x; i < CV_MAP; i += 64 * NW)
             sMap[i] = i < a.cvs.card ? a.cvs.map[i] : 0.0f;
     }
 
@@ -691,27 +691,29 @@ __global__ __launch_bounds__(64 * NW, 1) void k_phase1q(P1QueueArgs qa)
  * The SS table of a band comes from memory, which is why the rest, that fills
  * the chip, keeps its shared copy in LDS.  Without the bands a profile of
  * 3,000 columns against 1,337 rows was 6 stripes x 3,063 steps in one wave,
- * two waves on each SIMD: 12,000 profiles took 21.6 ms, now 15.9; with
- * context vectors, 181 rows x 6,000: 1.97 -> 1.65; 150 x 2,000: 0.88 -> 0.76 ms. */
-template <int R, int RB, int NW, bool CV>
+ * two waves on each SIMD: 12,000 profiles took 21.6 ms, now 15.9; 150 x
+ * 2,000: 0.88 -> 0.76 ms.  Not with context vectors: their wide columns leave
+ * one wave per SIMD, whose throughput is the bound (181 rows x 6,000 profiles
+ * 4.74 ms without bands, 4.80 with). */
+template <int R, int RB, int NW>
 __global__ __launch_bounds__(64 * NW, 1) void k_phase1_mix(P1Args a)
 {
     extern __shared__ float lds[];
     const int wv = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int b = (int)blockIdx.x;
     if (b >= a.nlong) {
-        p1_sweep<R, NW, false, CV, false, const P1Args>(a, a.nlong + (b - a.nlong) * NW + wv, lds, nullptr, 0);
+        p1_sweep<R, NW, false, false, false, const P1Args>(a, a.nlong + (b - a.nlong) * NW + wv, lds, nullptr, 0);
         return;
     }
     P1Band bd;
     bd.ns = a.bstripes; bd.nw = a.bwaves;
-    float* hand = lds + (size_t)bd.nw * (CV ? NS_CV : NS_TOP) * RING;
+    float* hand = lds + (size_t)bd.nw * NS_TOP * RING;
     bd.hout = hand + wv * 5 * HAND;
     bd.hin = hand + (wv > 0 ? wv - 1 : 0) * 5 * HAND;
     const int pb = a.seg_pb[b], pe = a.seg_pe[b];
     bd.cut = __builtin_amdgcn_readfirstlane((int)((int64_t)a.dist[pe - 1] + a.len[pe - 1] - (int64_t)a.dist[pb]));
     bd.start();
-    p1_sweep<RB, NW, false, CV, false, const P1Args, true>(a, b, lds, nullptr, 0, &bd);
+    p1_sweep<RB, NW, false, false, false, const P1Args, true>(a, b, lds, nullptr, 0, &bd);
 }
 
 /* the backtrack pass of a query of several stripes: a workgroup takes a
@@ -883,14 +885,13 @@ static hipError_t launch_nw(const P1Args& a, int R, int grid, size_t lds, hipStr
     return hipGetLastError();
 }
 
-static const void* phase1_mix_fn(int R, bool multi, int NW, bool cv)
+static const void* phase1_mix_fn(int R, bool multi, int NW)
 {
 #define C2_P1M(RR)                                                                                       \
     if (R == RR) {                                                                                       \
-        if (multi) return NW == 8 ? (const void*)k_phase1_mix<RR, RR, 8, false> : (const void*)k_phase1_mix<RR, RR, 4, false>; \
-        return NW == 8 ? (const void*)k_phase1_mix<RR, 1, 8, false> : (const void*)k_phase1_mix<RR, 1, 4, false>; \
+        if (multi) return NW == 8 ? (const void*)k_phase1_mix<RR, RR, 8> : (const void*)k_phase1_mix<RR, RR, 4>; \
+        return NW == 8 ? (const void*)k_phase1_mix<RR, 1, 8> : (const void*)k_phase1_mix<RR, 1, 4>; \
     }
-    if (cv) return R == 1 ? (const void*)k_phase1_mix<1, 1, 4, true> : (const void*)k_phase1_mix<2, 1, 4, true>;
     C2_P1M(1) C2_P1M(2) C2_P1M(3) C2_P1M(4) C2_P1M(5)
 #undef C2_P1M
     return nullptr;
@@ -898,19 +899,19 @@ static const void* phase1_mix_fn(int R, bool multi, int NW, bool cv)
 
 /* the sweep with bands for the long segments; false: none here (no stripes to
  * run side by side, or more than one round of them without a hand-off row) */
-static bool launch_mix(const P1Args& a0, int R, int NW, bool cv, size_t lds, hipStream_t stream, hipError_t* e)
+static bool launch_mix(const P1Args& a0, int R, int NW, size_t lds, hipStream_t stream, hipError_t* e)
 {
     P1Args a = a0;
     const bool multi = a.nstripes > 1;
     if (a.nlong <= 0 || a.nlong > a.nseg || (NW != 8 && NW != 4)) return false;
-    const int rb = multi && !cv ? R : 1;
+    const int rb = multi ? R : 1;
     a.bstripes = (a.Lq + 64 * rb - 1) / (64 * rb);
     if (a.bstripes < 2 || (!multi && a.bstripes > NW)) return false;
-    const void* fn = phase1_mix_fn(R, multi, NW, cv);
+    const void* fn = phase1_mix_fn(R, multi, NW);
     if (!fn) return false;
     const int rounds = (a.bstripes + NW - 1) / NW;
     a.bwaves = (a.bstripes + rounds - 1) / rounds;
-    const size_t bl = sizeof(float) * ((size_t)a.bwaves * ((cv ? NS_CV : NS_TOP) * RING + 5 * HAND) + (cv ? CV_MAP : 0));
+    const size_t bl = sizeof(float) * ((size_t)a.bwaves * (NS_TOP * RING + 5 * HAND));
     const int grid = a.nlong + (a.nseg - a.nlong + NW - 1) / NW;
     if (bl > lds) lds = bl;
     void* args[] = {&a};
@@ -929,7 +930,6 @@ hipError_t c2_launch_phase1(const P1Args& a, int R, int NW, bool btck, hipStream
         const int nw = btck ? 2 : 4;
         const int grid = (a.nseg + nw - 1) / nw;
         const size_t lds = phase1_cv_lds_bytes(R, nw);
-        if (!btck && launch_mix(a, R, nw, true, lds, stream, &e)) return e;
         if (btck) return R == 1 ? launch_cv<1, 2, true>(a, grid, lds, stream) : launch_cv<2, 2, true>(a, grid, lds, stream);
         return R == 1 ? launch_cv<1, 4, false>(a, grid, lds, stream) : launch_cv<2, 4, false>(a, grid, lds, stream);
     }
@@ -944,7 +944,7 @@ hipError_t c2_launch_phase1(const P1Args& a, int R, int NW, bool btck, hipStream
             default: return hipErrorInvalidValue;
         }
     }
-    if (!a.mfma && launch_mix(a, R, NW, false, lds, stream, &e)) return e;
+    if (!a.mfma && launch_mix(a, R, NW, lds, stream, &e)) return e;
     /* the DB sweep with the 20-term sums on the matrix cores */
     if (a.mfma) {
         switch (NW) {

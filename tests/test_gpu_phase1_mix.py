@@ -2,8 +2,8 @@
 the rest: these go to workgroups of their own whose waves take the query's
 stripes side by side.  Their maxima equal the oracle's and those of
 workgroups of one wave, which have no such bands, for every number of rows per
-lane, one to eleven stripes, with and without context vectors, and lengths
-around a refill and a hand-off ring."""
+lane, one to eleven stripes, and lengths around a refill and a hand-off ring.
+With context vectors there are no bands; the same databases are checked."""
 import numpy as np
 import pytest
 from comer2_amd._ffi import SynthDB
