@@ -826,7 +826,8 @@ extern "C" int cbp_sdp_prepare(cbp_handle* h, const cbp_sdp_pair* pairs, int32_t
     /* a workgroup's band: a pair's stripes, at most 4: two workgroups then
      * fit a CU with the adjoint's registers, and a pair of few stripes leaves
      * few wave slots idle (1,024 pairs of 50-600, a step: bands of 8 4.93 ms,
-     * 4 4.03; 24 pairs of 2,000-5,000 25.8 and 21.5) */
+     * 4 4.03; 24 pairs of 2,000-5,000 25.8 and 21.5; both sides with another
+     * form of the cells than the kernels have now, which take 3.9 and 22.2) */
     int maxL1 = 1;
     for (int32_t i = 0; i < npairs; i++) maxL1 = std::max(maxL1, (int)q.len[pairs[i].qidx]);
     const int nw = std::min(C2_SDP_BAND, (maxL1 + 63) / 64);

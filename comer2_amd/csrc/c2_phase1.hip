@@ -694,7 +694,7 @@ __global__ __launch_bounds__(64 * NW, 1) void k_phase1q(P1QueueArgs qa)
  * two waves on each SIMD: 12,000 profiles took 21.6 ms, now 15.9; 150 x
  * 2,000: 0.88 -> 0.76 ms.  Not with context vectors: their wide columns leave
  * one wave per SIMD, whose throughput is the bound (181 rows x 6,000 profiles
- * 4.74 ms without bands, 4.80 with). */
+ * 4.74-4.80 ms without bands, 4.80 with). */
 template <int R, int RB, int NW>
 __global__ __launch_bounds__(64 * NW, 1) void k_phase1_mix(P1Args a)
 {
