@@ -143,6 +143,8 @@ int cbp_destroy(cbp_handle* h)
         if (h->stage[s]) (void)hipHostFree(h->stage[s]);
         if (h->up_ev[s]) (void)hipEventDestroy(h->up_ev[s]);
     }
+    for (auto* v : {&h->sdp_uses, &h->sdp_capuses})
+        for (auto& u : *v) (void)hipEventDestroy(u.ev);
     if (h->ustream) (void)hipStreamDestroy(h->ustream);
     for (int s = 0; s < C2_NSTREAMS - 1; s++)
         if (h->xstream[s]) (void)hipStreamDestroy(h->xstream[s]);
@@ -796,6 +798,14 @@ static int sdp_upload_queries(cbp_handle* h)
     return CBP_OK;
 }
 
+/* the event of a workspace's last launch, recorded when first needed */
+static hipError_t sdp_recorded(cbp_handle::SdpUse& u)
+{
+    hipError_t e = hipSuccess;
+    if (!u.rec && (e = hipEventRecord(u.ev, u.st)) == hipSuccess) u.rec = true;
+    return e;
+}
+
 extern "C" int cbp_sdp_prepare(cbp_handle* h, const cbp_sdp_pair* pairs, int32_t npairs, int32_t ckpt,
                                int64_t* ws_bytes)
 {
@@ -806,6 +816,11 @@ extern "C" int cbp_sdp_prepare(cbp_handle* h, const cbp_sdp_pair* pairs, int32_t
     (void)hipSetDevice(h->device);
     h->sdp_ready = false;
     int rc;
+    /* the plan before this one is read by its launches */
+    for (auto& u : h->sdp_uses) {
+        HIPCHK(sdp_recorded(u));
+        HIPCHK(hipEventSynchronize(u.ev));
+    }
     if ((rc = sdp_upload_queries(h))) return rc;
     const cbp_profiles& q = h->queries.v;
     const cbp_profiles& d = h->chunk.v;
@@ -904,6 +919,75 @@ extern "C" int cbp_sdp_prepare(cbp_handle* h, const cbp_sdp_pair* pairs, int32_t
     return CBP_OK;
 }
 
+/* A launch keeps its item counter, the rows that its bands wait for and its
+ * sums in the workspace and starts by resetting them, so a launch that is
+ * still running there would lose rows that nobody writes again and wait for
+ * them without end.  Launches of this handle on overlapping workspaces
+ * therefore follow each other, whatever their streams: the new one's stream
+ * waits for the event of the last one there.  Launches that are being captured
+ * are ordered among those of the same capture (a replay is the caller's to
+ * order).  An event costs a small call 3-4 us (one pair of 40 x 40, a forward:
+ * 45 -> 48 us), so the default stream's, which outlives every call, is
+ * recorded only when another stream comes to wait for it.
+ *
+ * Before the launch: its stream waits for the workspace's last one */
+static int sdp_enter(cbp_handle* h, const void* ws, hipStream_t st, cbp_handle::SdpUse** use)
+{
+    const char* lo = (const char*)ws;
+    const char* hi = lo + h->sdp_ws_floats * (int64_t)sizeof(float);
+    hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+    unsigned long long id = 0;
+    /* (the default stream is never captured; a stream that cannot tell is
+     * taken for a direct one, and the launch reports what is wrong with it) */
+    if (st && hipStreamGetCaptureInfo(st, &cs, &id) != hipSuccess) {
+        (void)hipGetLastError();
+        cs = hipStreamCaptureStatusNone;
+    }
+    const bool cap = cs == hipStreamCaptureStatusActive;
+    if (cap && id != h->sdp_capid) {
+        for (auto& u : h->sdp_capuses) (void)hipEventDestroy(u.ev);
+        h->sdp_capuses.clear();
+        h->sdp_capid = id;
+    }
+    std::vector<cbp_handle::SdpUse>& v = cap ? h->sdp_capuses : h->sdp_uses;
+    /* of many workspaces those whose launches have ended are forgotten */
+    if (!cap && v.size() >= 8)
+        for (size_t i = v.size(); i-- > 0;) {
+            HIPCHK(sdp_recorded(v[i]));
+            if (hipEventQuery(v[i].ev) == hipSuccess) {
+                (void)hipEventDestroy(v[i].ev);
+                v.erase(v.begin() + i);
+            }
+        }
+    *use = nullptr;
+    for (auto& u : v) {
+        if (!(u.lo < hi && lo < u.hi)) continue;
+        /* one stream orders its launches by itself (a stream that a caller made
+         * may be another one of the same address by now, but not in a capture) */
+        if (!(u.st == st && (cap || !st))) {
+            HIPCHK(sdp_recorded(u));
+            HIPCHK(hipStreamWaitEvent(st, u.ev, 0));
+        }
+        if (u.lo == lo && u.hi == hi) *use = &u;
+    }
+    if (!*use) {
+        hipEvent_t ev = nullptr;
+        HIPCHK(hipEventCreateWithFlags(&ev, hipEventDisableTiming));
+        v.push_back({lo, hi, ev, st, true});
+        *use = &v.back();
+    }
+    return CBP_OK;
+}
+
+/* after it */
+static int sdp_leave(cbp_handle* h, cbp_handle::SdpUse* use, hipStream_t st)
+{
+    use->st = st;
+    use->rec = false;
+    if (st) HIPCHK(sdp_recorded(*use));
+    return CBP_OK;
+}
+
 static void sdp_fill(cbp_handle* h, SdpArgs* a, const float* S, const float* theta, void* ws, bool adjoint)
 {
     std::memset(a, 0, sizeof *a);
@@ -931,9 +1015,13 @@ extern "C" int cbp_sdp_forward(cbp_handle* h, const float* S, const float* theta
     SdpArgs a;
     sdp_fill(h, &a, S, theta, ws, false);
     a.logZ = logZ;
+    if (a.npairs <= 0) return CBP_OK;
+    cbp_handle::SdpUse* use;
+    const int rc = sdp_enter(h, ws, (hipStream_t)stream, &use);
+    if (rc) return rc;
     HIPCHK(c2_launch_sdp(a, false, h->sdp_groups, h->sdp_nw, h->sdp_xoff[0], h->sdp_xn[0],
                          (hipStream_t)stream));
-    return CBP_OK;
+    return sdp_leave(h, use, (hipStream_t)stream);
 }
 
 extern "C" int cbp_sdp_adjoint(cbp_handle* h, const float* S, const float* theta, const float* logZ,
@@ -946,9 +1034,13 @@ extern "C" int cbp_sdp_adjoint(cbp_handle* h, const float* S, const float* theta
     SdpArgs a;
     sdp_fill(h, &a, S, theta, ws, true);
     a.logZ = (float*)logZ; a.gZ = gZ; a.dS = dS; a.dth = dtheta; a.post = post;
+    if (a.npairs <= 0) return CBP_OK;
+    cbp_handle::SdpUse* use;
+    const int rc = sdp_enter(h, ws, (hipStream_t)stream, &use);
+    if (rc) return rc;
     HIPCHK(c2_launch_sdp(a, true, h->sdp_groups, h->sdp_nw, h->sdp_xoff[1], h->sdp_xn[1],
                          (hipStream_t)stream));
-    return CBP_OK;
+    return sdp_leave(h, use, (hipStream_t)stream);
 }
 
 extern "C" int cbp_sdp_scores(cbp_handle* h, float* S, void* stream)

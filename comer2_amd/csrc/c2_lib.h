@@ -321,6 +321,11 @@ struct cbp_handle {
     int32_t sdp_K = 0, sdp_nw = 1, sdp_groups = 1;
     int64_t sdp_ws_floats = 0, sdp_scr_off = 0;
     bool sdp_ready = false;
+    /* the last launch on each workspace: direct ones, and those of the capture
+     * sdp_capid; rec: the event has been recorded after it */
+    struct SdpUse { const char* lo; const char* hi; hipEvent_t ev; hipStream_t st; bool rec; };
+    std::vector<SdpUse> sdp_uses, sdp_capuses;
+    unsigned long long sdp_capid = 0;
 };
 
 /* internal helpers shared by the library's translation units */
