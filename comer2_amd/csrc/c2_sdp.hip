@@ -101,6 +101,7 @@ __device__ __forceinline__ void ld_trn(const float* T, int64_t ntr, int64_t base
  * words (clamped into the row when read). */
 typedef float f4u __attribute__((ext_vector_type(4), aligned(4)));
 typedef float f4 __attribute__((ext_vector_type(4)));
+typedef double f64u __attribute__((aligned(4)));
 
 __device__ __forceinline__ f4u grp_load(const float* row, int c0, int L2)
 {
@@ -293,7 +294,10 @@ __device__ __forceinline__ float* last_row(const SdpArgs& a, const SdpPair& P, i
                              : a.ws + P.hoff + (int64_t)s * 5 * P.L2;
 }
 
-/* four steps' states of the lane: a group's block is [5][64 lanes][4] */
+/* four steps' states of the lane: a group's block is [5][64 lanes][4].  The
+ * workspace is the caller's, at any float's address: its words are accessed
+ * as such (the device takes 16-byte accesses at 4-byte addresses, and no
+ * instruction differs for an aligned workspace) */
 struct Quad { f4 mm, mi, im, dn, nd; };
 __device__ __forceinline__ void quad_set(Quad& q, int u, const S5& s)
 {
@@ -306,12 +310,12 @@ __device__ __forceinline__ S5 quad_get(const Quad& q, int u)
 }
 __device__ __forceinline__ void quad_put(float* blk, int lane, const Quad& q)
 {
-    f4* p = (f4*)blk + lane;
+    f4u* p = (f4u*)blk + lane;
     p[0] = q.mm; p[64] = q.mi; p[128] = q.im; p[192] = q.dn; p[256] = q.nd;
 }
 __device__ __forceinline__ void quad_load(const float* blk, int lane, Quad& q)
 {
-    const f4* p = (const f4*)blk + lane;
+    const f4u* p = (const f4u*)blk + lane;
     q.mm = p[0]; q.mi = p[64]; q.im = p[128]; q.dn = p[192]; q.nd = p[256];
 }
 constexpr int QUAD = 5 * 64 * 4;      /* floats of a group's block */
@@ -783,7 +787,7 @@ __global__ __launch_bounds__(64 * C2_SDP_BAND) void k_sdp_adj(SdpArgs a)
         if (threadIdx.x < 5) {
             double t = 0.0;
             for (int k = 0; k < nwb; k++) t += wacc[k][threadIdx.x];
-            if (a.head) ((double*)(a.ws + a.dpart_off))[(int64_t)5 * (P.i0 + b) + threadIdx.x] = t;
+            if (a.head) ((f64u*)(a.ws + a.dpart_off))[(int64_t)5 * (P.i0 + b) + threadIdx.x] = t;
             else a.dth[(size_t)pi * 5 + threadIdx.x] = (float)(t * g);
         }
         __syncthreads();
@@ -805,7 +809,7 @@ __global__ __launch_bounds__(256) void k_sdp_sums(SdpArgs a, int adjoint)
     if (pi >= a.npairs) return;
     const SdpPair P = a.pairs[pi];
     if (adjoint) {
-        const double* d = (const double*)(a.ws + a.dpart_off) + (int64_t)5 * P.i0;
+        const f64u* d = (const f64u*)(a.ws + a.dpart_off) + (int64_t)5 * P.i0;
         const float g = a.gZ ? a.gZ[pi] : 1.0f;
         for (int j = 0; j < 5; j++) {
             double t = 0.0;

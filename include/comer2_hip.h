@@ -442,7 +442,8 @@ int  cbp_last_kernel_ms(const cbp_handle* h, double* ms, int32_t* nlaunch);
  * exp(F+B-logZ), the quantity of CuBatchMAPDP_bwd.cu:531-544.
  * S, theta, logZ, gZ, dS, dtheta, post and ws are device pointers; stream is
  * a hipStream_t (NULL: the default stream, which waits for the handle's own
- * stream and is waited for by it); calls are asynchronous.  A workspace holds
+ * stream and is waited for by it); calls are asynchronous.  Pointers need the
+ * alignment of a float, the workspace included.  A workspace holds
  * the state of one call at a time: calls of one handle on the same workspace
  * follow each other, on any streams, and calls on different workspaces may run
  * side by side.  What this cannot see is the caller's to order: replays of a

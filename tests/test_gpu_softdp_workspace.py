@@ -85,3 +85,20 @@ def test_captured_calls_on_two_streams():
         assert torch.equal(e, ref[rep % 3]), rep
         for t, r in zip((a, b, c), ref):
             assert torch.equal(t, r), rep
+
+
+@pytest.mark.parametrize("ckpt", [0, 32])
+def test_workspace_at_any_float(ckpt):
+    """a workspace that starts one, two or three floats into an allocation"""
+    import torch
+    cbp, sdp, ins, th, ref = _prepared(ckpt=ckpt)
+    z = sdp.forward(ins[0], th)
+    want = sdp.adjoint(ins[0], th, z, want_post=True)
+    room = torch.empty(sdp.ws.numel() + 3, dtype=torch.float32, device="cuda")
+    for off in (1, 2, 3):
+        print(f"workspace: {4 * off} bytes in, ckpt {ckpt}", flush=True)
+        sdp.ws = room[off:off + sdp.ws_bytes // 4]
+        z2 = sdp.forward(ins[0], th)
+        got = sdp.adjoint(ins[0], th, z2, want_post=True)
+        torch.cuda.synchronize()
+        assert torch.equal(z2, z) and all(torch.equal(x, y) for x, y in zip(got, want)), off
