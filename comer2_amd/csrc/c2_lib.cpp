@@ -369,11 +369,22 @@ SegSet* c2_segments(cbp_handle* h, int nq, int* rc)
 
 /* as many waves as the tuning and the LDS allow, but no more than spread the
  * segments over every CU: 150 segments in workgroups of 8 would keep 19 of
- * 256 CUs busy with two waves on each SIMD */
-int c2_phase1_waves(const cbp_handle* h, int R, int nstripes, int nseg)
+ * 256 CUs busy with two waves on each SIMD.  The matrix-core sweep has 8 or 4
+ * waves and keeps at least 4 */
+int c2_phase1_waves(const cbp_handle* h, int R, int nstripes, int nseg, bool mfma)
 {
     int nw = h->nw;
-    while (nw > 1 && (c2_phase1_lds_bytes(R, nw, nstripes) > 160 * 1024 || (int64_t)h->ncu * (nw / 2) >= nseg)) nw >>= 1;
+    const int least = mfma && nw >= 4 ? 4 : 1;
+    while (nw > least && (c2_phase1_lds_bytes(R, nw, nstripes) > 160 * 1024 || (int64_t)h->ncu * (nw / 2) >= nseg)) nw >>= 1;
+    return nw;
+}
+
+int c2_phase1_shape(cbp_handle* h, const QueryPrep& hp, P1Args* a)
+{
+    int nw = c2_phase1_waves(h, hp.R, hp.nstripes, a->nseg, a->mfma != 0);
+    if (a->cvs.wgt > 0.0f) { nw = 4; a->mfma = 0; }
+    if (nw < 4) a->mfma = 0;
+    h->last_p1_waves = nw; h->last_p1_mfma = a->mfma;
     return nw;
 }
 
@@ -620,7 +631,7 @@ int c2_run_phase1(cbp_handle* h, int qidx)
     if ((rc = dalloc(h, h->wts, sizeof(float) * 20 * (size_t)h->dchunk.nprof))) return rc;
     a.wts = h->wts.as<float>();
     HIPCHK(c2_launch_weights(dq->qbkg.as<float>(), h->dchunk.bkg.as<float>(), h->dchunk.nprof, h->wts.as<float>(), h->stream));
-    const int nw = c2_phase1_waves(h, dq->hp.R, dq->hp.nstripes, a.nseg);
+    const int nw = c2_phase1_shape(h, dq->hp, &a);
     HIPCHK(hipMemsetAsync(h->keys.p, 0, sizeof(unsigned long long) * h->dchunk.nprof, h->stream));
     HIPCHK(hipEventRecord(h->ev0, h->stream));
     HIPCHK(c2_launch_phase1(a, dq->hp.R, nw, false, h->stream));
@@ -651,6 +662,15 @@ int cbp_last_kernel_ms(const cbp_handle* h, double* ms, int32_t* nlaunch)
     if (!h || !ms) return CBP_ERR_ARG;
     *ms = h->last_ms;
     if (nlaunch) *nlaunch = h->last_nlaunch;
+    return CBP_OK;
+}
+
+int cbp_last_phase1_shape(const cbp_handle* h, int32_t* waves, int32_t* mfma)
+{
+    C2ApiScope c2_scope_;
+    if (!h || !waves || !mfma) return CBP_ERR_ARG;
+    *waves = h->last_p1_waves;
+    *mfma = h->last_p1_mfma;
     return CBP_OK;
 }
 

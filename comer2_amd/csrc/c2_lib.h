@@ -245,6 +245,7 @@ struct cbp_handle {
     int nw = 8;          /* tuning: waves per workgroup */
     double last_ms = 0.0;
     int32_t last_nlaunch = 0;
+    int32_t last_p1_waves = 0, last_p1_mfma = 0;   /* of the last one-query sweep */
     /* staged pipeline: per-query work, extra streams (default priority) and
      * one stripe hand-off buffer per stream */
     std::vector<std::unique_ptr<QWork>> work;
@@ -363,7 +364,10 @@ int c2_build_segments(cbp_handle* h, const cbp_profiles* s);
  * first use); null on failure */
 SegSet* c2_segments(cbp_handle* h, int nq, int* rc);
 /* waves per workgroup of a one-query launch over nseg segments */
-int c2_phase1_waves(const cbp_handle* h, int R, int nstripes, int nseg);
+int c2_phase1_waves(const cbp_handle* h, int R, int nstripes, int nseg, bool mfma);
+/* the same for the launch that a describes, with the context vectors' fixed
+ * shape; says whether the matrix cores are used and notes the shape */
+int c2_phase1_shape(cbp_handle* h, const QueryPrep& hp, P1Args* a);
 int c2_run_phase1(cbp_handle* h, int qidx);
 int c2_run_queries(cbp_handle* h, const int32_t* qidx, int32_t nq, const float* scorethld,
                    const float* logevthld, cbp_results* outs);

@@ -111,7 +111,7 @@ extern "C" int cbp_phase1_keys_noalloc(cbp_handle* h, int32_t qidx, uint64_t* ke
     a.seg_pb = g.db.as<int32_t>(); a.seg_pe = g.de.as<int32_t>(); a.nseg = g.nseg; a.nlong = g.nlong;
     a.keys = (unsigned long long*)(base + o_keys);
     a.bot = hp.nstripes > 1 ? (float*)(base + o_bot) : nullptr;
-    const int nw = c2_phase1_waves(h, hp.R, hp.nstripes, a.nseg);
+    const int nw = c2_phase1_waves(h, hp.R, hp.nstripes, a.nseg, false);
     /* the maxima start at zero (a kernel, not a memset) */
     if (c2_launch_zero_u64(a.keys, (int64_t)np, st) != hipSuccess ||
         c2_launch_weights(a.qbkg, a.bkg, (int)np, wts, st) != hipSuccess ||

@@ -74,7 +74,7 @@ int phase1_launch(cbp_handle* h, QWork& w, bool timed, bool copy = true)
     if ((rc = c2_fill_p1args(h, dq, &a))) return rc;
     a.keys = w.dk;
     if (dq->hp.nstripes > 1) a.bot = h->sbot[w.slot].as<float>();
-    const int nw = c2_phase1_waves(h, dq->hp.R, dq->hp.nstripes, a.nseg);
+    const int nw = c2_phase1_shape(h, dq->hp, &a);
     a.wts = w.dw;
     PCHK(c2_launch_zero_u64(w.dk, np, w.st));
     PCHK(c2_launch_weights(dq->qbkg.as<float>(), h->dchunk.bkg.as<float>(), np, w.dw, w.st));

@@ -43,6 +43,7 @@ def lib():
                                       C.POINTER(C.c_float), C.POINTER(C.c_float)]
     L.cbp_phase1_keys.argtypes = [H, C.c_int32, np.ctypeslib.ndpointer(np.uint64, flags="C")]
     L.cbp_last_kernel_ms.argtypes = [H, C.POINTER(C.c_double), C.POINTER(C.c_int32)]
+    L.cbp_last_phase1_shape.argtypes = [H, C.POINTER(C.c_int32), C.POINTER(C.c_int32)]
     L.cbp_set_tuning.argtypes = [H, C.c_int32, C.c_int32, C.c_int32]
     L.cbp_set_graph.argtypes = [H, C.c_int32]
     L.cbp_set_queue.argtypes = [H, C.c_int32]
@@ -197,6 +198,12 @@ class CuBatchProcessing:
         ms, n = C.c_double(), C.c_int32()
         self._check(self.L.cbp_last_kernel_ms(self.h, C.byref(ms), C.byref(n)))
         return ms.value, n.value
+
+    def last_phase1_shape(self):
+        """(waves per workgroup, matrix cores used) of the last one-query sweep"""
+        w, m = C.c_int32(), C.c_int32()
+        self._check(self.L.cbp_last_phase1_shape(self.h, C.byref(w), C.byref(m)))
+        return w.value, bool(m.value)
 
     def set_tuning(self, seg_cols=4096, rmax=5, nw=8):
         self._check(self.L.cbp_set_tuning(self.h, seg_cols, rmax, nw))

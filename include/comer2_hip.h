@@ -344,8 +344,9 @@ int  cbp_score_block(cbp_handle* h, int32_t qidx, int32_t pronr, float* S, float
 int  cbp_phase1_keys_noalloc(cbp_handle* h, int32_t qidx, uint64_t* keys /* [nprof] */);
 
 /* tuning of the phase-1 launch geometry: most DB columns per wave segment
- * (>= 64; smaller chunks are cut finer to fill the GPU), maximum query rows per lane (1..5) and waves per workgroup
- * (1, 2, 4, 8); no reference counterpart (the reference fixes 32x32 blocks,
+ * (>= 64; smaller chunks are cut finer to fill the GPU), maximum query rows
+ * per lane (1..5) and most waves per workgroup (1, 2, 4, 8; fewer when the
+ * chunk has too few segments to put such workgroups on every CU); no reference counterpart (the reference fixes 32x32 blocks,
  * cudp/CuBatchDP_com.h:16-30) */
 int  cbp_set_tuning(cbp_handle* h, int32_t seg_cols, int32_t rmax, int32_t nw);
 
@@ -385,7 +386,8 @@ int  cbp_set_queue(cbp_handle* h, int32_t on);
  * four columns with v_mfma_f32_4x4x1_16b_f32 chained over the 20 terms, one
  * product added per instruction, which rounds as the fmaf chain does, so
  * keys and every later stage are bit-identical.  The backtrack pass and the
- * context-vector sweep keep the vector form.  Replaces the score-matrix
+ * context-vector sweep keep the vector form, and so does a one-query launch
+ * tuned to fewer than 4 waves per workgroup.  Replaces the score-matrix
  * contraction of CalcSM_Init_SMEMUnroll2x (cusco/CuBatchScoreMatrix_Init.cu:45-186) */
 int  cbp_set_mfma(cbp_handle* h, int32_t on);
 
@@ -431,6 +433,10 @@ int  cbp_last_fallbacks(const cbp_handle* h, int32_t* n);
 /* device-side elapsed time of the last cbp_phase1_keys / cbp_process call's
  * dominant kernel (ms, HIP events on its stream) and the number of launches */
 int  cbp_last_kernel_ms(const cbp_handle* h, double* ms, int32_t* nlaunch);
+
+/* shape of the last one-query phase-1 sweep (cbp_phase1_keys, cbp_process):
+ * waves per workgroup, and whether the matrix cores formed the score sums */
+int  cbp_last_phase1_shape(const cbp_handle* h, int32_t* waves, int32_t* mfma);
 
 /* ---- differentiable soft DP (no reference counterpart) ----
  * The model is the MAP forward model of ExecMAPDP_Fwd_Unroll32x

@@ -86,3 +86,29 @@ def test_mfma_searches_equal_vector_sweep():
         assert _same(a, b)
     for a, b in zip(res[False][1], res[True][1]):
         assert _same(a, b)
+
+
+@pytest.mark.parametrize("nprof,nw", [(60, 8), (60, 4), (600, 8), (1400, 8)])
+def test_mfma_sweep_is_the_one_launched(nprof, nw):
+    """the matrix-core sweep runs whatever the number of segments (one or two
+    profiles each here), with 4 waves per workgroup or 8, and its keys are the
+    vector sweep's; one and two stripes, every rows-per-lane count"""
+    rng = np.random.default_rng(nprof)
+    q = SynthDB.from_lengths(511, [64, 100, 150, 230, 300, 330])
+    d = SynthDB.from_lengths(512, np.concatenate([rng.integers(64, 90, nprof - 50), rng.integers(20, 40, 50)]))
+    cbp = processing()
+    cbp.set_tuning(4096, 5, nw)
+    cbp.TransferQueries(q)
+    cbp.TransferCPMData(d)
+    for qp in range(q.nprof):
+        print(f"mfma launched: {nprof} profiles, nw={nw}, query {qp}", flush=True)
+        cbp.set_mfma(False)
+        ref = cbp.phase1_keys(qp)
+        assert not cbp.last_phase1_shape()[1]
+        cbp.set_mfma(True)
+        got = cbp.phase1_keys(qp)
+        waves, on = cbp.last_phase1_shape()
+        assert on and waves == (8 if nprof > 1100 else 4), (waves, on)
+        assert np.array_equal(got, ref)
+        res = cbp.ProcessScoreMatrix(qp, 6.0, math.log(1e-3))
+        assert cbp.last_phase1_shape() == (waves, True) and res["npassed"] >= 0
