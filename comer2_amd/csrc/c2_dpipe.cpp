@@ -49,13 +49,13 @@ DlCaps dl_caps(cbp_handle* h, const std::vector<int>& lq, const std::vector<int>
      * (stripes x (len + 63) x 64 each), so a small chunk holds a small pool */
     const int64_t allw = (int64_t)smax * ((int64_t)h->dchunk.npos + 63 * (int64_t)np) * 64;
     k.capW = std::max<int64_t>(64, std::min<int64_t>(h->dl_capW, allw));
-    c2_map_geometry(Lmax, &k.mR, &k.mns, &k.mnw);
+    c2_map_geometry(Lmax, h->map_pipe, &k.mR, &k.mns, &k.mnw);
     const int64_t chunks = (maxlen + C2_MAP_SCORE_COLS - 1) / C2_MAP_SCORE_COLS;
     int64_t cells = 0, hand = 0;
     int nsmax = 1;
     for (int L : lq) {
         int R = 1, ns = 1, nw = 1;
-        c2_map_geometry(L, &R, &ns, &nw);
+        c2_map_geometry(L, h->map_pipe, &R, &ns, &nw);
         nsmax = std::max(nsmax, ns);
         cells = std::max(cells, c2_map_cells(R, ns, maxlen));
         hand = std::max(hand, (c2_map_hand(ns, maxlen) + 63) & ~(int64_t)63);
@@ -208,7 +208,7 @@ int dl_chain(cbp_handle* h, int i, const DlPlan& P)
                          ahead ? sl.passfin.as<int32_t>() : nullptr, sl.statin.as<StatIn>(),
                          k.capP, sl.statout.as<double>(), st, q.cnt.as<int32_t>() + DL_NPASS));
     int mR = 1, mns = 1, mnw = 1;
-    c2_map_geometry(hp.Lq, &mR, &mns, &mnw);
+    c2_map_geometry(hp.Lq, h->map_pipe, &mR, &mns, &mnw);
     /* the shorter pairs of a split call: fewer, busier waves per pair */
     int mR2 = mR, mns2 = mns, mnw2 = mnw;
     if (P.split && h->map_rmax2 > 0) c2_map_geometry_short(hp.Lq, h->map_rmax2, &mR2, &mns2, &mnw2);

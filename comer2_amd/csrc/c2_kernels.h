@@ -202,8 +202,9 @@ hipError_t c2_dl_order_select(const double* statout, const DlBufs& b, const DlSe
 hipError_t c2_dl_aln_lists(const DlBufs& b, hipStream_t st);
 hipError_t c2_dl_results(const DlBufs& b, hipStream_t st);
 
-/* MAP geometry for a query: rows per lane and waves per pair */
-void c2_map_geometry(int Lq, int* R, int* ns, int* nw);
+/* MAP geometry for a query: rows per lane and waves per pair, in the streaming
+ * passes (pipe) or those of a workgroup per pair */
+void c2_map_geometry(int Lq, bool pipe, int* R, int* ns, int* nw);
 /* the geometry of the shorter pairs' group: at most rmax rows per lane, as
  * few stripes as that allows (fewer waves per pair, each busier) */
 void c2_map_geometry_short(int Lq, int rmax, int* R, int* ns, int* nw);

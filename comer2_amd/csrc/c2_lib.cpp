@@ -1157,7 +1157,7 @@ extern "C" int cbp_chunk_limits(cbp_handle* h, uint64_t qlen, uint64_t* maxpos, 
     int R = 1, ns = 1;
     c2_geometry((int)qlen, h->rmax, &R, &ns);
     int mR = 1, mns = 1, mnw = 1;
-    c2_map_geometry((int)qlen, &mR, &mns, &mnw);
+    c2_map_geometry((int)qlen, h->map_pipe, &mR, &mns, &mnw);
     /* phase 1, per DB position: 20 target frequencies, 3 SS probabilities,
      * 7 transitions, residue, SS state, profile index; the stripe hand-off
      * (5 floats) for multi-stripe queries; per profile: 20 background

@@ -1367,10 +1367,9 @@ hipError_t launch_r(const ScoreCtx& c, const MapArgs& m0, int npairs, hipStream_
     C2_LDS_LIMIT_ONCE(k_map_bwd_pipe<R>, 16 * 128 * MTW * sizeof(float));
     const int gf = pipe ? pipe_grid(k_map_fwd_pipe<R>, m.nw, npairs, lds) : npairs;
     const int gb = pipe ? pipe_grid(k_map_bwd_pipe<R>, m.nw, npairs, lds) : npairs;
-    const int wgb = wg > 512 ? 512 : wg;                              /* bands of the per-pair kernels */
     auto bwd = [&](hipStream_t st) {
         if (pipe) hipLaunchKernelGGL((k_map_bwd_pipe<R>), dim3(gb), dim3(wg), lds, st, c, m);
-        else hipLaunchKernelGGL((k_map_bwd<R>), dim3(npairs), dim3(wgb), 0, st, c, m);
+        else hipLaunchKernelGGL((k_map_bwd<R>), dim3(npairs), dim3(wg), 0, st, c, m);
     };
     if (bstream) {
         if ((e = hipEventRecord(fork, stream)) != hipSuccess) return e;
@@ -1379,7 +1378,7 @@ hipError_t launch_r(const ScoreCtx& c, const MapArgs& m0, int npairs, hipStream_
         if ((e = hipEventRecord(join, bstream)) != hipSuccess) return e;
     }
     if (pipe) hipLaunchKernelGGL((k_map_fwd_pipe<R>), dim3(gf), dim3(wg), lds, stream, c, m);
-    else hipLaunchKernelGGL((k_map_fwd<R>), dim3(npairs), dim3(wgb), 0, stream, c, m);
+    else hipLaunchKernelGGL((k_map_fwd<R>), dim3(npairs), dim3(wg), 0, stream, c, m);
     hipLaunchKernelGGL((k_map_total<R>), dim3(npairs), dim3(npairs > 1024 ? 256 : 1024), 0, stream, c, m);
     if (bstream) {
         if ((e = hipStreamWaitEvent(stream, join, 0)) != hipSuccess) return e;
@@ -1388,7 +1387,7 @@ hipError_t launch_r(const ScoreCtx& c, const MapArgs& m0, int npairs, hipStream_
     }
     if (pipe) hipLaunchKernelGGL((k_map_dp_pipe<R>), dim3(pipe_grid(k_map_dp_pipe<R>, m.nw, npairs, 0)), dim3(wg), 0,
                                  stream, c, m);
-    else hipLaunchKernelGGL((k_map_dp<R>), dim3(npairs), dim3(wgb), 0, stream, c, m);
+    else hipLaunchKernelGGL((k_map_dp<R>), dim3(npairs), dim3(wg), 0, stream, c, m);
     hipLaunchKernelGGL((k_map_final<R>), dim3(npairs), dim3(64), 0, stream, c, m, npairs);
     return hipGetLastError();
 }
@@ -1398,12 +1397,15 @@ hipError_t launch_r(const ScoreCtx& c, const MapArgs& m0, int npairs, hipStream_
 int64_t c2_map_cells(int R, int nstripes, int Ld) { return (int64_t)nstripes * (Ld + 63) * R * 64; }
 int64_t c2_map_hand(int nstripes, int Ld) { return (int64_t)nstripes * 5 * Ld + 4 * (int64_t)Ld; }
 
-/* one row per lane while a workgroup's 16 waves cover the query (a pair's
- * chain of steps is then the shortest), beyond 1,024 rows as many rows per
- * lane as let 8 waves cover it (R <= 5); waves = stripes of the first band */
-void c2_map_geometry(int Lq, int* R, int* ns, int* nw)
+/* streaming passes (pipe): one row per lane while a workgroup's 16 waves
+ * cover the query (a pair's chain of steps is then the shortest).  Beyond
+ * 1,024 rows, and in the passes of a workgroup per pair, whose bands have 8
+ * waves: as many rows per lane as let 8 waves cover it (R <= 5).  waves =
+ * stripes of the first band */
+void c2_map_geometry(int Lq, bool pipe, int* R, int* ns, int* nw)
 {
-    int r = Lq <= 1024 ? 1 : (Lq + 511) / 512;
+    int r = pipe && Lq <= 1024 ? 1 : (Lq + 511) / 512;
+    if (r < 1) r = 1;
     if (r > 5) r = 5;
     int n = (Lq + 64 * r - 1) / (64 * r);
     if (n < 1) n = 1;
@@ -1425,7 +1427,7 @@ hipError_t c2_launch_map(const ScoreCtx& c, const MapArgs& m, int npairs, hipStr
                          hipStream_t bstream, hipEvent_t fork, hipEvent_t join)
 {
     if (npairs <= 0) return hipSuccess;
-    if (m.nw < 1 || m.nw > (m.R == 1 ? 16 : 8) || m.ns < 1 || !m.order || !m.sitems || !m.B ||
+    if (m.nw < 1 || m.nw > (m.R == 1 && m.pipe ? 16 : 8) || m.ns < 1 || !m.order || !m.sitems || !m.B ||
         (!m.dcnt && m.nsitems < npairs * m.ns))
         return hipErrorInvalidValue;
     if (bstream && (!fork || !join)) return hipErrorInvalidValue;

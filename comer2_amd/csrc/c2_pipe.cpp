@@ -546,7 +546,7 @@ int stage_map(cbp_handle* h, QWork& w, bool split)
     if (nmap == 0) return CBP_OK;
     if (!h->opt.mapaln) return stage_aln(h, w);
     int mR = 1, mns = 1, mnw = 1;
-    c2_map_geometry(dq->hp.Lq, &mR, &mns, &mnw);
+    c2_map_geometry(dq->hp.Lq, h->map_pipe, &mR, &mns, &mnw);
     w.mp.resize(nmap);
     int64_t foff = 0, boff = 0, hoff = 0;
     int maxld = 0;

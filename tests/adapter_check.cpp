@@ -18,6 +18,9 @@
 #include <vector>
 #include "../include/hip_batch_processing.h"
 
+/* the library's own: rows per lane, stripes and waves of the MAP passes */
+void c2_map_geometry(int Lq, bool pipe, int* R, int* ns, int* nw);
+
 namespace {
 
 constexpr int NF = CBP_PM_NFIELDS;
@@ -186,5 +189,7 @@ int c2t_run(const cbp_profiles* qs, const cbp_profiles* db, int nsplit, const cb
         return e.code();
     }
 }
+
+void c2t_map_geometry(int lq, int pipe, int* out) { c2_map_geometry(lq, pipe != 0, out, out + 1, out + 2); }
 
 }  /* extern "C" */
