@@ -348,6 +348,7 @@ __global__ __launch_bounds__(BT) void k_dl_order_select(const double* statout, D
     /* offsets in launch order, each group with its geometry (the shorter
      * pairs' one when the call splits) */
     const int gR2 = sa.split ? sa.mR2 : sa.mR, gns2 = sa.split ? sa.mns2 : sa.mns;
+    const int ghand2 = sa.split ? sa.mhand2 : sa.mhand;
     int64_t cc = 0, hc = 0;
     for (int base = 0; base < nsel; base += BT) {
         const int o = base + threadIdx.x;
@@ -355,8 +356,9 @@ __global__ __launch_bounds__(BT) void k_dl_order_select(const double* statout, D
         const int k = ok ? b.morder[o] : 0;
         const int Ld = ok ? sa.len[b.mpairs[k].pro] : 0;
         const int gR = o < nA ? sa.mR : gR2, gns = o < nA ? sa.mns : gns2;
+        const int64_t grows = o < nA ? sa.mhand : ghand2;
         const int64_t cells = ok ? (int64_t)gns * (Ld + 63) * gR * 64 : 0;
-        const int64_t hand = ok ? ((int64_t)gns * 5 * Ld + 4 * (int64_t)Ld + 63) & ~(int64_t)63 : 0;
+        const int64_t hand = ok ? (grows * Ld + 63) & ~(int64_t)63 : 0;
         int64_t tc, th;
         const int64_t fo = cc + block_scan(cells, &tc);
         const int64_t ho = hc + block_scan(hand, &th);

@@ -35,6 +35,8 @@ struct DlCaps {
     int mR, mns, mnw;
 };
 
+int64_t hand_floats(int rows, int Ld) { return ((int64_t)rows * Ld + 63) & ~(int64_t)63; }
+
 DlCaps dl_caps(cbp_handle* h, const std::vector<int>& lq, const std::vector<int>& nstripes)
 {
     DlCaps k{};
@@ -58,12 +60,12 @@ DlCaps dl_caps(cbp_handle* h, const std::vector<int>& lq, const std::vector<int>
         c2_map_geometry(L, h->map_pipe, &R, &ns, &nw);
         nsmax = std::max(nsmax, ns);
         cells = std::max(cells, c2_map_cells(R, ns, maxlen));
-        hand = std::max(hand, (c2_map_hand(ns, maxlen) + 63) & ~(int64_t)63);
+        hand = std::max(hand, hand_floats(c2_map_hand_rows(h->map_pipe, ns, nw), maxlen));
         if (h->map_rmax2 > 0) {
             c2_map_geometry_short(L, h->map_rmax2, &R, &ns, &nw);
             nsmax = std::max(nsmax, ns);
             cells = std::max(cells, c2_map_cells(R, ns, maxlen));
-            hand = std::max(hand, (c2_map_hand(ns, maxlen) + 63) & ~(int64_t)63);
+            hand = std::max(hand, hand_floats(c2_map_hand_rows(h->map_pipe, ns, nw), maxlen));
         }
     }
     k.capItems = (int64_t)k.capM * nsmax * chunks;
@@ -219,6 +221,8 @@ int dl_chain(cbp_handle* h, int i, const DlPlan& P)
     sa.mapaln = h->opt.mapaln;
     sa.mR = mR; sa.mns = mns;
     sa.mR2 = mR2; sa.mns2 = mns2;
+    sa.mhand = c2_map_hand_rows(h->map_pipe, mns, mnw);
+    sa.mhand2 = c2_map_hand_rows(h->map_pipe, mns2, mnw2);
     sa.modinuse = (h->opt.ssswgt > 0.0f || h->opt.cvswgt > 0.0f) ? 1 : 0;
     sa.split = P.split ? 1 : 0;
     DCHK(c2_dl_order_select(sl.statout.as<double>(), b, sa, st));

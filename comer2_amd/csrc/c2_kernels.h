@@ -192,6 +192,7 @@ struct DlSelArgs {
     float logevthld;
     int32_t cap, mapaln, mR, mns, modinuse, split;
     int32_t mR2, mns2;     /* geometry of the shorter pairs' group (split calls) */
+    int32_t mhand, mhand2; /* hand-off rows of a pair, of a shorter one */
 };
 hipError_t c2_dl_candidates(const unsigned long long* keys, int32_t np, float thld, const DlBufs& b,
                             const int32_t* len, int32_t nstripes, P1Args* dargs, P1Tile* tiles, int32_t qslot,
@@ -214,9 +215,11 @@ void c2_map_geometry_short(int Lq, int rmax, int* R, int* ns, int* nw);
  * join are events of the handle (unused without bstream) */
 hipError_t c2_launch_map(const ScoreCtx& c, const MapArgs& m, int npairs, hipStream_t stream,
                          hipStream_t bstream, hipEvent_t fork, hipEvent_t join);
-/* floats of a pair's lane-step matrix (stripes x (Ld+63) steps x 64R) and of its hand-off buffers */
+/* floats of a pair's lane-step matrix (stripes x (Ld+63) steps x 64R) */
 int64_t c2_map_cells(int R, int nstripes, int Ld);
-int64_t c2_map_hand(int nstripes, int Ld);
+/* rows of Ld floats that a pair's bands hand over through memory: none when
+ * one band streams its pairs (its rows cross in LDS) */
+int c2_map_hand_rows(bool pipe, int nstripes, int nw);
 
 size_t c2_phase1_lds_bytes(int R, int NW, int nstripes);
 hipError_t c2_launch_zero_u64(unsigned long long* p, int64_t n, hipStream_t stream);

@@ -1395,7 +1395,7 @@ hipError_t launch_r(const ScoreCtx& c, const MapArgs& m0, int npairs, hipStream_
 }  // namespace
 
 int64_t c2_map_cells(int R, int nstripes, int Ld) { return (int64_t)nstripes * (Ld + 63) * R * 64; }
-int64_t c2_map_hand(int nstripes, int Ld) { return (int64_t)nstripes * 5 * Ld + 4 * (int64_t)Ld; }
+int c2_map_hand_rows(bool pipe, int nstripes, int nw) { return pipe && nw == nstripes ? 0 : nstripes * 5 + 4; }
 
 /* streaming passes (pipe): one row per lane while a workgroup's 16 waves
  * cover the query (a pair's chain of steps is then the shortest).  Beyond

@@ -547,6 +547,7 @@ int stage_map(cbp_handle* h, QWork& w, bool split)
     if (!h->opt.mapaln) return stage_aln(h, w);
     int mR = 1, mns = 1, mnw = 1;
     c2_map_geometry(dq->hp.Lq, h->map_pipe, &mR, &mns, &mnw);
+    const int hrows = c2_map_hand_rows(h->map_pipe, mns, mnw);
     w.mp.resize(nmap);
     int64_t foff = 0, boff = 0, hoff = 0;
     int maxld = 0;
@@ -566,7 +567,7 @@ int stage_map(cbp_handle* h, QWork& w, bool split)
         const int64_t cells = c2_map_cells(mR, mns, ch.len[p]);
         foff += cells;
         boff += cells;
-        hoff += (c2_map_hand(mns, ch.len[p]) + 63) & ~(int64_t)63;
+        hoff += ((int64_t)hrows * ch.len[p] + 63) & ~(int64_t)63;
         if (ch.len[p] > maxld) maxld = ch.len[p];
     }
     /* launch order: longest DB profile first (ties by selection order) */

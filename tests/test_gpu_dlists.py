@@ -108,3 +108,22 @@ def test_device_lists_per_query_launches_fresh_handle():
     host = cbp.ProcessBatch(qs)
     for i in qs:
         _same(dev[i], host[i], ("per-query launches", i))
+
+
+def test_streamed_map_bands_need_no_hand_off_rows():
+    """900 rows x 2,000 drawn profiles of 500: the streaming passes cross their
+    rows in LDS, so only the matrices bound what the device lists take"""
+    q = SynthDB.from_lengths(451, [900])
+    d = SynthDB.from_lengths(452, [500] * 2000)
+    cbp = processing(dict(max_map_pairs=0))
+    cbp.set_device_list_caps(4096, 4096, 1 << 30, 1 << 31)
+    cbp.TransferQueries(q)
+    cbp.TransferCPMData(d)
+    cbp.SetDbDetails(d.npos, d.nprof)
+    print("device lists: 900 x 2,000 pairs", flush=True)
+    res = cbp.ProcessScoreMatrix(0, scorethld=-1.0, logevthld=50.0)
+    assert res["nmap"] > 1900 and cbp.last_fallbacks() == 0
+    cbp.set_device_lists(False)
+    host = cbp.ProcessScoreMatrix(0, scorethld=-1.0, logevthld=50.0)
+    for k in ("alndata", "order", "aln_raw"):
+        assert np.ascontiguousarray(res[k]).tobytes() == np.ascontiguousarray(host[k]).tobytes(), k
