@@ -128,8 +128,8 @@ __global__ __launch_bounds__(256) void k_dl_cand_scatter(const unsigned long lon
 }
 
 /* backtrack-code offsets of the candidates (words: stripes x (len + 63) x
- * 64 each), the backtrack pass's segment count and its queue tiles (pairs of
- * candidates) */
+ * 64 each), the backtrack pass's segment count and, unless it takes them one
+ * by one (no tiles), its queue tiles (pairs of candidates) */
 __global__ __launch_bounds__(BT) void k_dl_cand_prep(const int32_t* len, const int32_t* cand, int32_t nstripes,
                                                     int64_t* off, int64_t capW, int32_t* cnt,
                                                     P1Args* args, P1Tile* tiles, int32_t qslot, int32_t* ntiles)
@@ -146,7 +146,7 @@ __global__ __launch_bounds__(BT) void k_dl_cand_prep(const int32_t* len, const i
         carry += tot;
     }
     const bool wovf = carry > capW;
-    const int ng = (ovf || wovf) ? 0 : (nc + 1) / 2;
+    const int ng = (ovf || wovf || !tiles) ? 0 : (nc + 1) / 2;
     for (int g = threadIdx.x; g < ng; g += BT) tiles[g] = P1Tile{qslot, g};
     if (threadIdx.x == 0) {
         off[nc] = carry;

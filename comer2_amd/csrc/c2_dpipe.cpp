@@ -170,9 +170,9 @@ int dl_chain(cbp_handle* h, int i, const DlPlan& P)
     const QueryPrep& hp = w.dq->hp;
     DCHK(c2_launch_zero_u32((uint32_t*)q.cnt.p, DL_NCNT, st));
     DCHK(c2_dl_candidates(w.dk, d.nprof, w.scorethld, b, d.len.as<int32_t>(), hp.nstripes, q.dargs.as<P1Args>(),
-                          q.tiles.as<P1Tile>(), 0, q.ntiles.as<int32_t>(), st));
-    /* the backtrack pass: the query's candidates from its queue, in pairs, or
-     * one by one when a candidate's stripes run in a band of waves */
+                          hp.nstripes > 1 ? nullptr : q.tiles.as<P1Tile>(), 0, q.ntiles.as<int32_t>(), st));
+    /* the backtrack pass: the query's candidates from its queue, in pairs
+     * (tiles), or one by one when a candidate's stripes run in a band of waves */
     P1QueueArgs qa;
     qa.args = q.dargs.as<P1Args>();
     qa.tiles = q.tiles.as<P1Tile>();
@@ -376,12 +376,15 @@ int c2_run_queries_dev(cbp_handle* h, const int32_t* qidx, int32_t nq, const flo
     for (int i = 0; i < nq; i++) {
         QWork& w = *h->work[i];
         const QueryPrep& hp = w.dq->hp;
-        const size_t lds = c2_phase1_lds_bytes(hp.R, 2, hp.nstripes);
-        if (lds > 80 * 1024) return c2_fail(h, CBP_ERR_STATE, "backtrack pass exceeds the LDS");
-        P.lds[i] = lds;
-        P.grid[i] = hp.nstripes > 1 ? c2_btck_band_grid(hp.R, hp.nstripes) : c2_phase1q_grid(hp.R, 2, true, lds);
+        if (hp.nstripes > 1) {
+            P.grid[i] = c2_btck_band_grid(hp.R, hp.nstripes);
+            botw = std::max<int64_t>(botw, (int64_t)P.grid[i] * 5 * h->chunk_maxlen);
+        } else {
+            P.lds[i] = c2_phase1_lds_bytes(hp.R, 2, 1);
+            if (P.lds[i] > 80 * 1024) return c2_fail(h, CBP_ERR_STATE, "backtrack pass exceeds the LDS");
+            P.grid[i] = c2_phase1q_grid(hp.R, 2, true, P.lds[i]);
+        }
         if (P.grid[i] < 1) return c2_fail(h, CBP_ERR_HIP, "backtrack queue occupancy");
-        if (hp.nstripes > 1) botw = std::max<int64_t>(botw, (int64_t)P.grid[i] * 5 * h->chunk_maxlen);
         uint64_t delta = 0;
         w.sspace = c2_length_adjustment(h->opt, (uint64_t)hp.Lq, dblen, nseqs, &delta);
         StatParams& sp = P.sp[i];

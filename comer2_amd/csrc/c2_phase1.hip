@@ -885,14 +885,15 @@ static hipError_t launch_nw(const P1Args& a, int R, int grid, size_t lds, hipStr
     return hipGetLastError();
 }
 
+/* (a query of several stripes has at most 4 rows per lane: c2_geometry) */
 static const void* phase1_mix_fn(int R, bool multi, int NW)
 {
-#define C2_P1M(RR)                                                                                       \
-    if (R == RR) {                                                                                       \
-        if (multi) return NW == 8 ? (const void*)k_phase1_mix<RR, RR, 8> : (const void*)k_phase1_mix<RR, RR, 4>; \
-        return NW == 8 ? (const void*)k_phase1_mix<RR, 1, 8> : (const void*)k_phase1_mix<RR, 1, 4>; \
+#define C2_P1M(RR, RB) if (R == RR) return NW == 8 ? (const void*)k_phase1_mix<RR, RB, 8> : (const void*)k_phase1_mix<RR, RB, 4>;
+    if (multi) {
+        C2_P1M(1, 1) C2_P1M(2, 2) C2_P1M(3, 3) C2_P1M(4, 4)
+    } else {
+        C2_P1M(2, 1) C2_P1M(3, 1) C2_P1M(4, 1) C2_P1M(5, 1)
     }
-    C2_P1M(1) C2_P1M(2) C2_P1M(3) C2_P1M(4) C2_P1M(5)
 #undef C2_P1M
     return nullptr;
 }
@@ -989,7 +990,6 @@ static const void* btck_band_fn(int R)
         case 2: return (const void*)k_btck_band<2>;
         case 3: return (const void*)k_btck_band<3>;
         case 4: return (const void*)k_btck_band<4>;
-        case 5: return (const void*)k_btck_band<5>;
         default: return nullptr;
     }
 }

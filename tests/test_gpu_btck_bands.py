@@ -2,8 +2,8 @@
 side by side in a band of up to four waves, in rounds, and give the records
 and alignments of one wave taking the stripes in turn (the host-decided
 lists), bit for bit; profile lengths around a refill, the waves' distance and
-a hand-off ring, 2 to 5 stripes and more, 1 to 5 rows per lane, and more
-candidates than workgroups."""
+a hand-off ring, 2 to 5 stripes and more, 1 to 4 rows per lane (a query of
+several stripes has no more), and more candidates than workgroups."""
 import numpy as np
 import pytest
 from comer2_amd._ffi import SynthDB
