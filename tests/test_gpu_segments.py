@@ -76,3 +76,30 @@ def test_segment_arrays_are_kept_between_chunks():
         one = [cbp.ProcessScoreMatrix(i) for i in range(2)]
         for i, r in enumerate(cbp.ProcessBatch([0, 1] * nq)):
             assert np.array_equal(r["alndata"].view(np.uint32), one[i % 2]["alndata"].view(np.uint32)), (nq, i)
+
+
+# 4 and 8 waves per workgroup over segments of several profiles (two or three,
+# and about six), none of them long: 513-1,024 segments and more
+@pytest.mark.parametrize("nprof,hi,waves", [(1700, 40, 4), (3600, 40, 8), (14000, 120, 8)])
+@pytest.mark.parametrize("lq,rmax", [(60, 1), (100, 1), (120, 5), (200, 2), (180, 5), (340, 5), (250, 5), (500, 5), (310, 5)])
+def test_segments_of_several_profiles(lq, rmax, nprof, hi, waves):
+    rng = np.random.default_rng(nprof)
+    lens = rng.integers(24, hi + 1, nprof)
+    q = SynthDB.from_lengths(241, [lq])
+    d = SynthDB.from_lengths(242, lens)
+    print(f"segments of several: Lq={lq} rmax={rmax} nprof={nprof}", flush=True)
+    cbp = processing()
+    cbp.set_tuning(4096, rmax, 8)
+    cbp.TransferQueries(q)
+    cbp.TransferCPMData(d)
+    keys = cbp.phase1_keys(0)
+    assert cbp.last_phase1_shape() == (waves, False)
+    orc = oracle()
+    from comer2_amd.host import encode_key
+    for dp in [int(i) for i in np.linspace(0, nprof - 1, 60)]:
+        S, _ = orc.score_f32(q.view, 0, d.view, dp)
+        m, _, _ = orc.viterbi_f32(q.view, 0, d.view, dp, S)
+        assert int(keys[dp]) == encode_key(m.maxsc, m.x, m.y), (lq, rmax, dp, int(lens[dp]))
+    cbp.set_tuning(4096, rmax, 1)
+    assert np.array_equal(keys, cbp.phase1_keys(0))
+    assert cbp.last_phase1_shape() == (1, False)
