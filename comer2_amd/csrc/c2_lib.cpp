@@ -301,7 +301,7 @@ static int64_t seg_target(const cbp_handle* h, int64_t npos, int nq)
 
 static int build_segset(cbp_handle* h, const cbp_profiles* s, int64_t target, SegSet* g)
 {
-    g->target = 0;
+    g->target = target;
     std::vector<std::pair<int32_t, int32_t>> v;
     int64_t acc = 0;
     int32_t p0 = 0;
@@ -334,21 +334,18 @@ static int build_segset(cbp_handle* h, const cbp_profiles* s, int64_t target, Se
     if ((rc = dupload(h, g->db, g->b.data(), g->b.size()))) return rc;
     if ((rc = dupload(h, g->de, g->e.data(), g->e.size()))) return rc;
     HIPCHK(hipStreamSynchronize(h->stream));
-    g->target = target;
     return CBP_OK;
 }
 
 /* a new chunk's (or a new tuning's) segments: the one-query set now, the
- * batches' when first used.  The sets keep their device arrays: freeing one
- * waits for every stream, and a streamed search comes here for each chunk
- * while the next one is copied */
+ * batches' when first used */
 int c2_build_segments(cbp_handle* h, const cbp_profiles* s)
 {
-    for (auto& g : h->segs) g->target = 0;
+    h->segs.clear();
     h->chunk_maxlen = 0;
     for (int32_t p = 0; p < s->nprof; p++)
         if (s->len[p] > h->chunk_maxlen) h->chunk_maxlen = s->len[p];
-    if (h->segs.empty()) h->segs.emplace_back(new SegSet());
+    h->segs.emplace_back(new SegSet());
     return build_segset(h, s, seg_target(h, s->npos, 1), h->segs[0].get());
 }
 
@@ -357,19 +354,17 @@ SegSet* c2_segments(cbp_handle* h, int nq, int* rc)
     *rc = CBP_OK;
     const int64_t target = seg_target(h, h->dchunk.npos, nq);
     for (auto& g : h->segs) if (g->target == target) return g.get();
-    size_t i = 1;
-    while (i < h->segs.size() && h->segs[i]->target) i++;
-    if (i == h->segs.size() && i >= 8) {
-        /* batches of many sizes: the oldest set goes, with the graphs that may
-         * hold its addresses */
+    /* batches of many sizes: the oldest set goes, with the graphs that may
+     * hold its addresses */
+    if (h->segs.size() >= 8) {
         (void)hipStreamSynchronize(h->stream);
         c2_drop_graphs(h);
-        std::rotate(h->segs.begin() + 1, h->segs.begin() + 2, h->segs.end());
-        i--;
+        h->segs.erase(h->segs.begin() + 1);
     }
-    if (i == h->segs.size()) h->segs.emplace_back(new SegSet());
-    if ((*rc = build_segset(h, &h->chunk.v, target, h->segs[i].get()))) return nullptr;
-    return h->segs[i].get();
+    std::unique_ptr<SegSet> g(new SegSet());
+    if ((*rc = build_segset(h, &h->chunk.v, target, g.get()))) return nullptr;
+    h->segs.push_back(std::move(g));
+    return h->segs.back().get();
 }
 
 /* as many waves as the tuning and the LDS allow, but no more than spread the

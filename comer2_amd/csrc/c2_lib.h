@@ -189,7 +189,7 @@ struct DlResult {
 /* the chunk cut into segments of whole profiles, the unit of work of one
  * phase-1 wave, widest first */
 struct SegSet {
-    int64_t target = 0;                 /* columns a segment aims at (0: of an earlier chunk) */
+    int64_t target = 0;                 /* columns a segment aims at */
     std::vector<int32_t> b, e;          /* first profile, one past the last */
     int32_t nseg = 0, maxcols = 0;      /* segments, columns of the widest */
     int32_t nlong = 0;                  /* leading segments swept by a workgroup each */

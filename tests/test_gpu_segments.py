@@ -54,30 +54,6 @@ def test_segment_order_and_batches(order):
         assert int(keys[dp]) == encode_key(m.maxsc, m.x, m.y), (order, dp)
 
 
-def test_segment_arrays_are_kept_between_chunks():
-    """a smaller chunk takes the device arrays of the chunk before: nothing is
-    freed, so the limits (the budget minus what is held) stay, and the larger
-    one fits them again"""
-    q = SynthDB.from_lengths(231, [90, 150])
-    big, small = SynthDB.from_lengths(232, [60] * 2500), SynthDB.from_lengths(233, [60] * 300)
-    from comer2_amd.host import CuBatchProcessing
-    cbp = CuBatchProcessing(0, mem_budget=6 << 30)
-    cbp.TransferQueries(q)
-    lim = []
-    for d in (big, small, big, small):
-        cbp.TransferCPMData(d)
-        cbp.SetDbDetails(d.npos, d.nprof)
-        print(f"segment arrays: {d.nprof} profiles", flush=True)
-        cbp.ProcessBatch([0, 1])
-        cbp.phase1_keys(0)
-        lim.append(cbp.chunk_limits(150))
-    assert len(set(lim)) == 1, lim
-    for nq in range(2, 14):                   # more batch sizes than sets are kept
-        one = [cbp.ProcessScoreMatrix(i) for i in range(2)]
-        for i, r in enumerate(cbp.ProcessBatch([0, 1] * nq)):
-            assert np.array_equal(r["alndata"].view(np.uint32), one[i % 2]["alndata"].view(np.uint32)), (nq, i)
-
-
 # 4 and 8 waves per workgroup over segments of several profiles (two or three,
 # and about six), none of them long: 513-1,024 segments and more
 @pytest.mark.parametrize("nprof,hi,waves", [(1700, 40, 4), (3600, 40, 8), (14000, 120, 8)])
