@@ -79,3 +79,22 @@ def test_segments_of_several_profiles(lq, rmax, nprof, hi, waves):
     cbp.set_tuning(4096, rmax, 1)
     assert np.array_equal(keys, cbp.phase1_keys(0))
     assert cbp.last_phase1_shape() == (1, False)
+
+
+def test_more_batch_sizes_than_segment_sets_are_kept():
+    """every size of batch cuts this chunk differently; eight sets are kept, and
+    replayed batches meet sets made anew"""
+    q = SynthDB.from_lengths(251, [60, 70])
+    d = SynthDB.from_lengths(252, [200] * 1500)
+    d.plant(q, 253, 8, 3.0, 60.0)
+    cbp = processing(dict(max_map_pairs=8))
+    cbp.TransferQueries(q)
+    cbp.TransferCPMData(d)
+    cbp.SetDbDetails(d.npos, d.nprof)
+    one = [cbp.ProcessScoreMatrix(i) for i in range(2)]
+    cbp.set_graph(True)
+    for nq in list(range(4, 16)) + [4, 4, 4, 9, 9, 9, 4]:
+        print(f"segment sets: batch of {nq}", flush=True)
+        for i, r in enumerate(cbp.ProcessBatch([k % 2 for k in range(nq)])):
+            assert np.array_equal(r["alndata"].view(np.uint32), one[i % 2]["alndata"].view(np.uint32)), (nq, i)
+            assert np.array_equal(r["aln_raw"], one[i % 2]["aln_raw"]), (nq, i)
