@@ -725,7 +725,7 @@ __global__ __launch_bounds__(64 * NW, 1) void k_phase1_mix(P1Args a)
  * slots in its ring of 64.  A round of nw stripes starts when wave 0 is done
  * with the round before (period: its blocks, at least 3 nw), and its first
  * stripe reads the last wave's row, kept in memory, three blocks behind it.
- * Up to BAND_MAX waves: 15 KB of LDS each, so several workgroups share a CU
+ * Up to BAND_MAX waves: 16 KB of LDS each, so several workgroups share a CU
  * and a list of many short candidates keeps the CU as busy as before; the
  * stripes are dealt evenly to the rounds (6: 3 and 3).  Bound by the longest
  * candidate's chain of steps.  1,337 rows in 6 stripes, candidates of up to

@@ -34,12 +34,16 @@
  * each K-step segment from its checkpoint into per-wave scratch and sweeps
  * it backwards (sqrt(L) checkpointing).
  *
- * What bounds it: VALU issue and the sweep's chain of steps.  Per cell 15
- * (forward) and 21 (adjoint) transcendentals at a quarter of the VALU rate and
- * about 75 and 110 other operations.  A step waits for no memory: a profile's
- * transitions pass through LDS, scores, stored states and gradients go four
- * columns at a time, and the terms that leave the matrix's edges are added
- * after the sweep.  One row per lane: the padding of a pair's last stripe is
+ * What bounds it: the sweep's chain of dependent steps, with too few waves to
+ * hide it.  Per cell 16 (forward) and 21 (adjoint) transcendentals, of two
+ * issue slots each, and about 115 and 155 other vector instructions; counted
+ * on 1,024 pairs of 50-600, the vector units are busy 38% (forward) and 31%
+ * (adjoint) of the time, with 2.6 and 1.8 waves per SIMD that spend 71% of
+ * theirs waiting; on 24 pairs of 2,000-5,000 with checkpoints 19% and 17%,
+ * with 0.8 waves.  No step loads what it uses: a profile's transitions pass
+ * through LDS, scores, stored states and gradients go four columns at a time
+ * a group ahead, and the terms that leave the matrix's edges are added after
+ * the sweep.  One row per lane: the padding of a pair's last stripe is
  * at most 63 rows, and a step's chain is one cell.  Every cell's operations
  * and their order are those of the one-workgroup-per-pair sweep.  Measured
  * (before: stripes of 320 rows, one workgroup per pair, inputs loaded in the

@@ -395,9 +395,10 @@ int  cbp_set_mfma(cbp_handle* h, int32_t on);
  * run as their own group beside the long pairs): rmax = 1..5 gives that
  * group at most rmax query rows per lane and as few stripes (waves per pair)
  * as that allows, so each wave works on more rows and fewer waves wait at
- * the band's per-step barriers; rmax = 0 keeps the long pairs' geometry
+ * the band's barriers (one per four steps when it streams its pairs, else one
+ * per step); rmax = 0 keeps the long pairs' geometry
  * (one row per lane in up to 16 waves for queries of at most 1,024 positions,
- * else up to 8 waves of R = ceil(Lq/512)) for every pair.  Results are
+ * else, and with streaming off, up to 8 waves of R = ceil(Lq/512)) for every pair.  Results are
  * bit-identical either way.  Replaces the fixed 32x32-block schedule of
  * ExecMAPDP_Parent_DynPlm (cumapdp/CuBatchMAPDP_prnt.cu:18-115) */
 int  cbp_set_map_rows(cbp_handle* h, int32_t rmax);
