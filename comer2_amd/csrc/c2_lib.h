@@ -277,7 +277,7 @@ struct cbp_handle {
      * geometry for every pair) */
     int map_rmax2 = 0;
     /* MAP forward and backward passes stream a workgroup's pairs through one
-     * band (queries whose stripes fit 8 waves) */
+     * band (queries whose stripes fit it: 16 waves at one row per lane, else 8) */
     bool map_pipe = true;
     QPlan qscan, qcand;
     DBuf qkeys, qwts;                   /* [nq][nprof] maxima, [nq][nprof][20] weights */

@@ -29,8 +29,8 @@ def _planted_sets(seed, qlen=None):
     return q, d
 
 
-# query lengths 60-400: one band of 1-7 stripes of 64 rows; 560-640: stripes
-# of 128 rows; 2600-2700: 320-row stripes in two bands (HBM band hand-off)
+# query lengths 60-400: one band of 1-7 stripes of 64 rows; 560-640: 9-10
+# stripes; 2600-2700: 320-row stripes in two bands (HBM band hand-off)
 @pytest.mark.parametrize("seed,cap,qlen", [(41, 0, None), (51, 5, None), (61, 6, (560, 640)),
                                            (71, 4, (2600, 2700))])
 def test_map_matches_oracle(seed, cap, qlen):

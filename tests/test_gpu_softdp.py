@@ -65,8 +65,8 @@ def test_soft_dp_matches_fp64_oracle(ckpt):
 
 @pytest.mark.parametrize("ckpt", [0, 32])
 def test_soft_dp_two_bands(ckpt):
-    """A 2,600-2,700-row query is nine 320-row stripes: two bands of waves,
-    the second fed through the HBM hand-off."""
+    """A 2,600-2,700-row query is 41 to 43 stripes: eleven bands of four waves,
+    all but the first fed through the hand-off rows in memory."""
     import torch
     from comer2_amd.softdp import SoftDP
     q = SynthDB(91, 1, 0, 0, 2600, 2700)

@@ -23,7 +23,7 @@ def _noalloc(cbp, qidx, nprof):
 
 def test_noalloc_keys_equal_phase1_keys():
     q = SynthDB(2302, 3, 0, 0, 150, 150)                 # three queries of 150
-    q2 = SynthDB(2305, 1, 0, 0, 700, 700)                # two stripes of 320 rows (R = 5)
+    q2 = SynthDB(2305, 1, 0, 0, 700, 700)                # three stripes of 256 rows (R = 4)
     big = SynthDB(2303, 3000, 200, 0.668, 30, 3000)
     small = SynthDB(2304, 500, 150, 0.668, 30, 800)
     cbp = processing()
